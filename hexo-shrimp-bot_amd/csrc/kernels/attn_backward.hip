@@ -2,9 +2,7 @@
 // operators (the reference's register_autograd pairs):
 //
 //  * typed segment attention (cell_attention / cell_attention_plain,
-//    python/mantisnet/mantisnet/cell_latents.py:570-621, 680-797), and the
-//    window-latent read and broadcast, which are the same attention over
-//    other edge lists (window_latents.py:132-230, 503-551).  With
+//    python/mantisnet/mantisnet/cell_latents.py:570-621, 680-797).  With
 //      score_e = scale q[qid_e] . k[src_e] + bias[cls_e]
 //      alpha_e = exp(score_e - m[qid_e]) / l[qid_e]        (the forward's softmax)
 //      dalpha_e = go[qid_e] . (v[src_e] + vcls[cls_e])

@@ -6,8 +6,9 @@ surface runs unchanged.  Each has a fake (meta) implementation for tracing.
 Every differentiable operator carries the reference's backward
 (``register_autograd`` with the reference's ``*_backward`` operators where it
 registers them): the run reductions and the cell pass as run reductions, the
-attention family and the window latents through one segment-attention
-backward (query-major pass, source-major pass, sliced class sums), the
+typed attentions through one segment-attention backward (query-major pass,
+source-major pass, sliced class sums), the window latents through a pass over
+the window rows each, the
 action-row encoder through masked run sums.  Every backward sums in a fixed
 order: two calls agree bitwise.
 
@@ -431,7 +432,7 @@ def window_latent_read_backward(q: Tensor, k: Tensor, v: Tensor, window_pos: Ten
                                 out: Tensor, m: Tensor, l: Tensor,
                                 grad_out: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     """(dq, dk, dv) of window_latent_read."""
-    return ops.latent_read_backward(q, k, v, window_pos, offsets, order, m, l, grad_out)
+    return ops.latent_read_backward(q, k, v, window_pos, offsets, order, out, m, l, grad_out)
 
 
 @window_latent_read_backward.register_fake

@@ -649,44 +649,56 @@ def attention_backward(q: Tensor, k: Tensor, v: Tensor, bias: Tensor | None, vcl
     return dq.view(q.shape), dk.view(k.shape), dv.view(v.shape), dbias, dvcls
 
 
-def _run_edges(offsets: Tensor, order: Tensor, slots: int):
-    """Row-major edge lists of 'every one of `slots` rows of position p meets
-    every window of p': per row p*slots+s the CSR of order[offsets[p]:offsets[p+1]]."""
-    cnt = (offsets[1:] - offsets[:-1]).repeat_interleave(slots)
-    ptr = torch.zeros(cnt.numel() + 1, dtype=torch.int64, device=offsets.device)
-    torch.cumsum(cnt, 0, out=ptr[1:])
-    rows = torch.repeat_interleave(torch.arange(cnt.numel(), device=offsets.device), cnt)
-    within = torch.arange(rows.numel(), device=offsets.device) - ptr[rows]
-    return ptr, order.index_select(0, offsets.index_select(0, rows // slots) + within)
+def _latent_rows(t: Tensor, rows: int, name: str) -> tuple[Tensor, int]:
+    """(rows, 128) view of latent or window rows, and its row stride."""
+    return _rows128(t if t.shape[0] == rows else t.reshape(rows, 128), name)
 
 
-def _slot_edges(window_pos: Tensor, slots: int):
-    """Row-major edge lists of 'window w meets the `slots` latent rows of its position'."""
-    n = window_pos.numel()
-    ptr = torch.arange(0, slots * n + 1, slots, dtype=torch.int64, device=window_pos.device)
-    dst = (window_pos.repeat_interleave(slots) * slots
-           + torch.arange(slots, device=window_pos.device).repeat(n))
-    return ptr, dst
+def _latent_backward(q, k, v, n_q, n_k, window_pos, offsets, order, m, l, grad_out, out):
+    dev = _on_gpu(q, k, v, window_pos, offsets, order, m, l, grad_out, out)
+    if k.dtype != q.dtype or v.dtype != q.dtype:
+        raise ValueError("q, k and v must share one dtype")
+    (q2, ldq), (k2, ldk), (v2, ldv) = (_latent_rows(t, n, s) for t, n, s in ((q, n_q, "q"), (k, n_k, "k"),
+                                                                             (v, n_k, "v")))
+    window_pos, offsets, order = _i64(window_pos, "window_pos"), _i64(offsets, "offsets"), _i64(order, "order")
+    n_pos, n_w = offsets.numel() - 1, window_pos.numel()
+    if n_pos < 0 or order.numel() != n_w or (n_q, n_k) != ((4 * n_pos, n_w) if out is not None else (n_w, 4 * n_pos)):
+        raise ValueError("offsets must be (P + 1,), order and window_pos (N_w,)")
+    go, m32, l32 = grad_out.reshape(n_q, 128).float().contiguous(), *(t.reshape(n_q, 4).float().contiguous()
+                                                                      for t in (m, l))
+    dq, dk, dv = (torch.empty((n, 128), dtype=q.dtype, device=dev) for n in (n_q, n_k, n_k))
+    ws = _workspace(_lib().mantis_latent_backward_workspace(n_pos, n_w), dev)
+    # the window rows and their gradients once, the fp32 gradient rows once
+    nbytes = (n_q + 2 * n_k) * 256 * q.element_size() + n_q * 128 * 4
+    flops = n_w * 4 * 128 * 10
+    if out is not None:
+        o32 = out.reshape(n_q, 128).float().contiguous()
+        _launch("latent_read_backward", nbytes, flops, lambda: _check(
+            _lib().mantis_latent_read_backward(
+                _ptr(q2), _ptr(k2), _ptr(v2), _dt(q), ldq, ldk, ldv, _ptr(window_pos), _ptr(offsets), _ptr(order),
+                n_pos, n_w, _ptr(go), _ptr(o32), _ptr(m32), _ptr(l32), _ptr(ws), ws.numel(), _ptr(dq), _ptr(dk),
+                _ptr(dv), _ptr(error_flag(dev)), _stream()),
+            "latent_read_backward"))
+    else:
+        _launch("latent_broadcast_backward", nbytes, flops, lambda: _check(
+            _lib().mantis_latent_broadcast_backward(
+                _ptr(q2), _ptr(k2), _ptr(v2), _dt(q), ldq, ldk, ldv, _ptr(window_pos), _ptr(offsets), _ptr(order),
+                n_pos, n_w, _ptr(go), _ptr(m32), _ptr(l32), _ptr(ws), ws.numel(), _ptr(dq), _ptr(dk), _ptr(dv),
+                _ptr(error_flag(dev)), _stream()),
+            "latent_broadcast_backward"))
+    return dq.view(q.shape), dk.view(k.shape), dv.view(v.shape)
 
 
-def latent_read_backward(q, k, v, window_pos, offsets, order, m, l, grad_out):
+def latent_read_backward(q, k, v, window_pos, offsets, order, out, m, l, grad_out):
     """(dq, dk, dv) of latent_read: the four slot queries of each position
-    over its windows (window_latents.py:132-163)."""
-    p_ptr, p_src = _run_edges(offsets, order, 4)
-    w_ptr, w_dst = _slot_edges(window_pos, 4)
-    dq, dk, dv, _, _ = attention_backward(q.reshape(-1, 4, 32), k, v, None, None, grad_out, m, l, p_ptr, p_src, None,
-                                          None, w_ptr, w_dst, None, None, None)
-    return dq.view(q.shape), dk, dv
+    over its windows (window_latents.py:132-163); out, m and l the forward's."""
+    return _latent_backward(q, k, v, q.shape[0] * 4, k.shape[0], window_pos, offsets, order, m, l, grad_out, out)
 
 
 def latent_broadcast_backward(q, k, v, window_pos, offsets, order, m, l, grad_out):
     """(dq, dk, dv) of latent_broadcast: every window over its position's four
     latent rows (window_latents.py:191-230)."""
-    w_ptr, w_dst = _slot_edges(window_pos, 4)
-    p_ptr, p_src = _run_edges(offsets, order, 4)
-    dq, dk, dv, _, _ = attention_backward(q, k.reshape(-1, 4, 32), v.reshape(-1, 4, 32), None, None, grad_out, m, l,
-                                          w_ptr, w_dst, None, None, p_ptr, p_src, None, None, None)
-    return dq, dk.view(k.shape), dv.view(v.shape)
+    return _latent_backward(q, k, v, q.shape[0], k.shape[0] * 4, window_pos, offsets, order, m, l, grad_out, None)
 
 
 def stone_attention_backward(q, k, v, seq_lens, out, lse, grad_out):

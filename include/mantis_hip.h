@@ -260,9 +260,7 @@ int32_t mantis_class_reduce(const void* values, int32_t values_dtype, int64_t n_
  * cptr, cedge_q, dbias_t); vcls NULL: no class values.  workspace: at least
  * mantis_attention_backward_workspace(n_q, n_entries, n_classes or 0) bytes.
  * Replaces mantisnet::cell_attention_backward / cell_attention_plain_backward
- * (python/mantisnet/mantisnet/cell_latents.py:570-621, 680-797, 869-1001) and
- * mantisnet::window_latent_read_backward / window_latent_broadcast_backward
- * (window_latents.py:132-230, 503-551, 589-712).
+ * (python/mantisnet/mantisnet/cell_latents.py:570-621, 680-797, 869-1001).
  */
 int64_t mantis_attention_backward_workspace(int64_t n_q, int64_t n_entries, int64_t n_classes);
 int32_t mantis_attention_backward(const void* q, const void* k, const void* v, int32_t dtype, int64_t ldq, int64_t ldk,
@@ -273,6 +271,33 @@ int32_t mantis_attention_backward(const void* q, const void* k, const void* v, i
                                   const int64_t* sqid, const int64_t* scls, const int64_t* cptr,
                                   const int64_t* cedge_q, void* workspace, int64_t workspace_bytes, void* dq,
                                   void* dk, void* dv, float* dbias_t, void* dvcls, int32_t* err_flag, void* stream);
+
+/*
+ * Backward of the window-latent read (latent queries q (4 n_pos rows) over
+ * window keys and values k, v (n_w rows)) and broadcast (window queries q
+ * over latent keys and values), rows of 4 heads x 32 in dtype with strides
+ * ldq / ldk / ldv (multiples of 8, at least 128).  offsets / order: the
+ * position-major window layout, window_pos each window's position.  grad_out
+ * (and, for the read, the forward's out) fp32 contiguous rows of q's count;
+ * m, l (rows of q, 4) the forward's softmax statistics.  dq, dk and dv
+ * contiguous in dtype.  One pass over the window rows and a merge; fp32 sums
+ * in a fixed order.  workspace: mantis_latent_backward_workspace(n_pos, n_w)
+ * bytes, 16-byte aligned.  Replaces the backward of
+ * mantisnet::window_latent_read / window_latent_broadcast
+ * (window_latents.py:132-230, 503-551, 589-712).
+ */
+int64_t mantis_latent_backward_workspace(int64_t n_pos, int64_t n_w);
+int32_t mantis_latent_read_backward(const void* q, const void* k, const void* v, int32_t dtype, int64_t ldq,
+                                    int64_t ldk, int64_t ldv, const int64_t* window_pos, const int64_t* offsets,
+                                    const int64_t* order, int64_t n_pos, int64_t n_w, const float* grad_out,
+                                    const float* out, const float* m, const float* l, void* workspace,
+                                    int64_t workspace_bytes, void* dq, void* dk, void* dv, int32_t* err_flag,
+                                    void* stream);
+int32_t mantis_latent_broadcast_backward(const void* q, const void* k, const void* v, int32_t dtype, int64_t ldq,
+                                         int64_t ldk, int64_t ldv, const int64_t* window_pos, const int64_t* offsets,
+                                         const int64_t* order, int64_t n_pos, int64_t n_w, const float* grad_out,
+                                         const float* m, const float* l, void* workspace, int64_t workspace_bytes,
+                                         void* dq, void* dk, void* dv, int32_t* err_flag, void* stream);
 
 /*
  * Backward of the action-row encoder: with mask_e = pre[edge_window[e]] +

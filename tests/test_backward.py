@@ -108,6 +108,64 @@ def test_window_latent_backward(device, batch):
     mantisnet.ops.raise_on_device_error(device)
 
 
+@pytest.mark.parametrize("counts,dt,shuffled", [
+    ([0], torch.float32, False), ([1], torch.float32, False), ([63, 64, 65], torch.float32, True),
+    ([3, 0, 700, 17], torch.float32, True), ([130, 1, 0], torch.bfloat16, False), ([16, 15, 257], torch.float16, True),
+])
+def test_window_latent_backward_layouts(device, counts, dt, shuffled):
+    """Runs around the lane groups and the split of a position's windows,
+    positions without windows, and windows whose order is not the identity."""
+    p, n_w = len(counts), sum(counts)
+    gen = torch.Generator().manual_seed(25 + n_w)
+    window_pos = torch.repeat_interleave(torch.arange(p), torch.tensor(counts))
+    if shuffled:
+        window_pos = window_pos[torch.randperm(n_w, generator=gen)]
+    offsets, order = R.window_layout(window_pos, p)
+    layout = [x.to(device) for x in (window_pos, offsets, order)]
+    shapes = [(p, 4, 4, 32), (n_w, 4, 32)]
+    for read in (True, False):
+        sq, sk = shapes if read else shapes[::-1]
+        q, k, v = (torch.randn(*s, generator=gen).to(dt) for s in (sq, sk, sk))
+        seed = torch.randn(*sq, generator=gen)
+        op = OPS.window_latent_read if read else OPS.window_latent_broadcast
+        got = _grads(lambda a, c, d: op(a, c, d, *layout)[0], [x.to(device) for x in (q, k, v)], seed.to(device))
+        ref = (lambda a, c, d: R.latent_read(a, c, d, offsets, order)) if read else (
+            lambda a, c, d: R.latent_broadcast(a, c, d, window_pos))
+        exp = _grads(ref, [x.float() for x in (q, k, v)], seed) if n_w else [torch.zeros(s) for s in (sq, sk, sk)]
+        _close(got, exp, dt)
+        assert all(g.dtype == dt for g in got)
+    mantisnet.ops.raise_on_device_error(device)
+
+
+def test_window_latent_backward_takes_any_order(device):
+    """An order that is not a permutation: the latent rows sum over the order's
+    runs, the window rows come from each window's own position."""
+    gen = torch.Generator().manual_seed(26)
+    window_pos = torch.tensor([0, 1, 1, 0, 1])
+    offsets, order = torch.tensor([0, 3, 5]), torch.tensor([0, 0, 2, 1, 4])  # window 3 unnamed, 0 twice, 2 misplaced
+    layout = [x.to(device) for x in (window_pos, offsets, order)]
+    q, k, v = (torch.randn(*s, generator=gen).to(device) for s in ((2, 4, 4, 32), (5, 4, 32), (5, 4, 32)))
+    go = torch.randn(2, 4, 4, 32, generator=gen).to(device)
+    out, m, l = OPS.window_latent_read(q, k, v, *layout)
+    dq, dk, dv = OPS.window_latent_read_backward(q, k, v, *layout, out, m, l, go)
+    sc = 32 ** -0.5
+    delta = (go * out).sum(-1)
+
+    def terms(w, p):  # alpha, dscore: (slots, heads)
+        al = torch.exp((q[p] * k[w]).sum(-1) * sc - m[p]) / l[p]
+        return al, al * ((go[p] * v[w]).sum(-1) - delta[p])
+
+    for p in range(2):
+        exp = sum(terms(w, p)[1][..., None] * k[w] * sc for w in order[offsets[p]:offsets[p + 1]].tolist())
+        torch.testing.assert_close(dq[p], exp, rtol=1e-4, atol=1e-4)
+    for w in range(5):
+        p = int(window_pos[w])
+        al, ds = terms(w, p)
+        torch.testing.assert_close(dv[w], (al[..., None] * go[p]).sum(0), rtol=1e-4, atol=1e-4)
+        torch.testing.assert_close(dk[w], (ds[..., None] * q[p]).sum(0) * sc, rtol=1e-4, atol=1e-4)
+    mantisnet.ops.raise_on_device_error(device)
+
+
 def test_action_row_encode_backward(device, batch):
     b = batch
     n_w, n_c = b.window_feat.numel(), b.cell_pos.shape[0]
