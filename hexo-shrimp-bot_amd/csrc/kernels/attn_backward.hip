@@ -186,13 +186,18 @@ attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_
   store8(dv + row * kRow + c0, gvv);
 }
 
-// dvcls slices: partial[s] = sum over the class-major entries j of slice s
-// of alpha[E, head] * go[qid[E]], E = cedge[j] (a query-major edge)
+// Class slices: partial4[s] = sum over the class-major entries j of slice s of
+// dscore[E], E = cedge[j] (a query-major edge), and with kV partial[s] = sum
+// of alpha[E, head] * go[qid[E]].  16 entries per index load; the gradient
+// rows of kLook entries in flight, the scores one entry per lane.  Bound by
+// the gathered gradient rows.
+template <bool kV>
 __global__ void __launch_bounds__(kBlock)
-vcls_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ go, int64_t ldgo,
-                  const int64_t* __restrict__ qid, int64_t n_q, const int64_t* __restrict__ cedge, int64_t n_edges,
-                  const int64_t* __restrict__ slice_edge, int64_t n_slices, float* __restrict__ partial,
-                  int32_t* flag) {
+class_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ dscore_e,
+                   const float* __restrict__ go, int64_t ldgo, const int64_t* __restrict__ qid, int64_t n_q,
+                   const int64_t* __restrict__ cedge, int64_t n_edges, const int64_t* __restrict__ slice_edge,
+                   int64_t n_slices, float* __restrict__ partial, float* __restrict__ partial4, int32_t* flag) {
+  constexpr int kLook = 4;
   const int64_t s = int64_t(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
   const int lane = threadIdx.x % kGroup;
   if (s >= n_slices) return;
@@ -201,24 +206,52 @@ vcls_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ g
   int64_t st, en;
   segment(slice_edge, s, n_edges, st, en);
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int64_t j = st; j < en; ++j) {
-    const int64_t E = cedge[j];
-    const int64_t qi = (E >= 0 && E < n_edges) ? qid[E] : -1;
-    if (qi < 0 || qi >= n_q) {
-      if (lane == 0) raise_flag(flag, MANTIS_FLAG_INDEX);
-      continue;
+  float4 d4 = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int64_t base = st; base < en; base += kGroup) {
+    const int cnt = int(en - base < kGroup ? en - base : kGroup);
+    const int64_t E = cedge[base + (lane < cnt ? lane : cnt - 1)];
+    bool ok = E >= 0 && E < n_edges;
+    int64_t qi = 0;
+    if (ok && lane < cnt) {
+      const float4 d = *reinterpret_cast<const float4*>(dscore_e + E * kHeads);
+      d4.x += d.x, d4.y += d.y, d4.z += d.z, d4.w += d.w;
     }
-    const float al = alpha_e[E * kHeads + h];
-    float gv[8];
-    load8(go + qi * ldgo + c0, gv);
+    if constexpr (kV) {
+      qi = ok ? qid[E] : -1;
+      ok = qi >= 0 && qi < n_q;
+    }
+    if (!ok && lane < cnt) raise_flag(flag, MANTIS_FLAG_INDEX);
+    if constexpr (kV) {
+      const int64_t row = ok ? qi : -1;
+      for (int j = 0; j < cnt; j += kLook) {
+        float gv[kLook][8], al[kLook];
+        bool use[kLook];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = fmaf(al, gv[i], acc[i]);
+        for (int u = 0; u < kLook; ++u) {
+          const int from = j + u < cnt ? j + u : cnt - 1;
+          const int64_t r = __shfl(row, from, kGroup), e = __shfl(E, from, kGroup);
+          use[u] = j + u < cnt && r >= 0;
+          if (use[u]) {  // uniform over the group
+            load8(go + r * ldgo + c0, gv[u]);
+            al[u] = alpha_e[e * kHeads + h];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kLook; ++u)
+          if (use[u])
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i] = fmaf(al[u], gv[u][i], acc[i]);
+      }
+    }
   }
-  store8(partial + s * kRow + c0, acc);
+  if constexpr (kV) store8(partial + s * kRow + c0, acc);
+  d4.x = row16_sum(d4.x), d4.y = row16_sum(d4.y), d4.z = row16_sum(d4.z), d4.w = row16_sum(d4.w);
+  if (lane == 0) *reinterpret_cast<float4*>(partial4 + s * kHeads) = d4;
 }
 
 // Row-encoder gradient runs: out[d] = sum over j in [ptr[d], ptr[d+1]) of
 // mask_E * go[cell_E], E = perm[j] (an entry of the cell-major decoder list).
+// 16 entries per index load, the rows of kLook entries in flight.
 template <typename Tp, typename Tt, typename To>
 __global__ void __launch_bounds__(kBlock)
 row_mask_kernel(const Tp* __restrict__ pre, int64_t ldp, int64_t n_w, const Tt* __restrict__ table, int64_t n_cls,
@@ -226,6 +259,7 @@ row_mask_kernel(const Tp* __restrict__ pre, int64_t ldp, int64_t n_w, const Tt* 
                 const int64_t* __restrict__ edge_class, const int64_t* __restrict__ edge_cell, int64_t n_edges,
                 const int64_t* __restrict__ ptr, const int64_t* __restrict__ perm, int64_t n_dest,
                 To* __restrict__ out, int32_t* flag) {
+  constexpr int kLook = 4;
   const int64_t d = int64_t(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
   const int lane = threadIdx.x % kGroup;
   if (d >= n_dest) return;
@@ -233,20 +267,35 @@ row_mask_kernel(const Tp* __restrict__ pre, int64_t ldp, int64_t n_w, const Tt* 
   int64_t st, en;
   segment(ptr, d, n_edges, st, en);
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int64_t j = st; j < en; ++j) {
-    const int64_t E = perm[j];
+  for (int64_t base = st; base < en; base += kGroup) {
+    const int cnt = int(en - base < kGroup ? en - base : kGroup);
+    const int64_t E = perm[base + (lane < cnt ? lane : cnt - 1)];
     const bool in = E >= 0 && E < n_edges;
     const int64_t w = in ? edge_window[E] : -1, c = in ? edge_class[E] : -1, cell = in ? edge_cell[E] : -1;
-    if (w < 0 || w >= n_w || c < 0 || c >= n_cls || cell < 0 || cell >= n_cells) {
-      if (lane == 0) raise_flag(flag, MANTIS_FLAG_INDEX);
-      continue;
-    }
-    float pv[8], tv[8], gv[8];
-    load8(pre + w * ldp + c0, pv);
-    load8(table + c * kRow + c0, tv);
-    load8(go + cell * kRow + c0, gv);
+    const bool good = w >= 0 && w < n_w && c >= 0 && c < n_cls && cell >= 0 && cell < n_cells;
+    if (!good && lane < cnt) raise_flag(flag, MANTIS_FLAG_INDEX);
+    for (int j = 0; j < cnt; j += kLook) {
+      Chunk8<Tp> pv[kLook];
+      Chunk8<Tt> tv[kLook];
+      Chunk8<float> gv[kLook];
+      bool use[kLook];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] += (pv[i] + tv[i] > 0.f) ? gv[i] : 0.f;
+      for (int u = 0; u < kLook; ++u) {
+        const int from = j + u < cnt ? j + u : cnt - 1;
+        const int64_t wu = __shfl(w, from, kGroup), cu = __shfl(c, from, kGroup), du = __shfl(cell, from, kGroup);
+        use[u] = __shfl(int(good), from, kGroup) != 0 && j + u < cnt;
+        if (use[u]) {  // uniform over the group
+          pv[u].load(pre + wu * ldp + c0);
+          tv[u].load(table + cu * kRow + c0);
+          gv[u].load(go + du * kRow + c0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kLook; ++u)
+        if (use[u])
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i] += (pv[u][i] + tv[u][i] > 0.f) ? gv[u][i] : 0.f;
+    }
   }
   store8(out + d * kRow + c0, acc);
 }
@@ -360,17 +409,13 @@ int32_t mantis_attention_backward(const void* q, const void* k, const void* v, i
   slice_edges_kernel<<<unsigned((S.n_slices + 1 + 255) / 256), 256, 0, s>>>(cptr, slice_ptr, n_classes, n_entries,
                                                                              S.n_slices, slice_edge);
   if ((st = launched()) != MANTIS_OK) return st;
-  st = mantis_run_reduce(dscore_e, MANTIS_F32, n_entries, kHeads, kHeads, cedge_q, n_entries, slice_edge, S.n_slices,
-                         partial4, MANTIS_F32, err_flag, stream);
-  if (st != MANTIS_OK) return st;
-  st = mantis_run_reduce(partial4, MANTIS_F32, S.n_slices, kHeads, kHeads, nullptr, S.n_slices, slice_ptr, n_classes,
-                         dbias_t, MANTIS_F32, err_flag, stream);
-  if (st != MANTIS_OK || !vcls) return st;
-  vcls_slice_kernel<<<grid_rows(S.n_slices), kBlock, 0, s>>>(alpha_e, grad_out, ldgo, qid, n_q, cedge_q, n_entries,
-                                                              slice_edge, S.n_slices, partial, err_flag);
+  auto slices = vcls ? class_slice_kernel<true> : class_slice_kernel<false>;
+  slices<<<grid_rows(S.n_slices), kBlock, 0, s>>>(alpha_e, dscore_e, grad_out, ldgo, qid, n_q, cedge_q, n_entries,
+                                                  slice_edge, S.n_slices, partial, partial4, err_flag);
   if ((st = launched()) != MANTIS_OK) return st;
-  return mantis_run_reduce(partial, MANTIS_F32, S.n_slices, kRow, kRow, nullptr, S.n_slices, slice_ptr, n_classes,
-                           dvcls, vcls_dtype, err_flag, stream);
+  st = slice_merge(partial4, kHeads, slice_ptr, S.n_slices, n_classes, dbias_t, s);
+  if (st != MANTIS_OK || !vcls) return st;
+  return slice_merge(partial, kRow, slice_ptr, S.n_slices, n_classes, dvcls, vcls_dtype, s);
 }
 
 int64_t mantis_row_encode_backward_workspace(int64_t n_entries, int64_t n_classes) {
@@ -419,8 +464,7 @@ int32_t mantis_row_encode_backward(const void* pre, int32_t pre_dtype, int64_t l
           static_cast<const Tp*>(pre), ldp, n_w, static_cast<const Tt*>(table), n_cls, grad_out, n_cells,
           edge_window, edge_class, edge_cell, n_entries, slice_edge, cls_order, S.n_slices, partial, err_flag);
       if ((st = launched()) != MANTIS_OK) return;
-      st = mantis_run_reduce(partial, MANTIS_F32, S.n_slices, kRow, kRow, nullptr, S.n_slices, slice_ptr, n_cls, dtable,
-                             table_dtype, err_flag, stream);
+      st = slice_merge(partial, kRow, slice_ptr, S.n_slices, n_cls, dtable, table_dtype, s);
       ok_o = st != MANTIS_E_ARG;
     });
   });

@@ -128,7 +128,8 @@ run_reduce_kernel(const Tin* __restrict__ values, int64_t n_src, int64_t ld, int
   constexpr int kLook = 4;
   // every lane runs every chunk step (the shuffles need all 16 lanes); a lane
   // past the row's width only skips its loads and its store
-  for (int64_t cb = 0; cb < h; cb += kGroup * 8) {
+  // (128 columns per grid row: the chunks of a wide row run side by side)
+  for (int64_t cb = int64_t(blockIdx.y) * (kGroup * 8); cb < h; cb += int64_t(gridDim.y) * (kGroup * 8)) {
     const int64_t c0 = cb + int64_t(lane) * 8;
     const bool mine = c0 < h;
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -864,7 +865,7 @@ int32_t mantis_run_reduce(const void* values, int32_t values_dtype, int64_t n_sr
                                          block, 0, s>>>(static_cast<const TI*>(values), n_src, ld, gather, ptr,
                                                         n_dest, n_entries, static_cast<TO*>(out), err_flag);
       else if (vec)
-        run_reduce_kernel<TI, TO><<<grid, block, 0, s>>>(static_cast<const TI*>(values), n_src, ld,
+        run_reduce_kernel<TI, TO><<<dim3(grid.x, unsigned(std::min<int64_t>((h + 127) / 128, 65535))), block, 0, s>>>(static_cast<const TI*>(values), n_src, ld,
                                                          h, gather, ptr, n_dest, n_entries,
                                                          static_cast<TO*>(out), err_flag);
       else

@@ -16,8 +16,8 @@
 // the ReLU mask, in the same loop that sums the gradient rows.  The window
 // sums are the library's run reduction.  Class runs can hold tens of
 // thousands of entries, so d_emb is two-level: every class run is cut into
-// slices of at most kSlice entries (one 16-lane group each), and a second
-// run reduction sums each class's slice partials in slice order.
+// slices of at most kSlice entries (one 16-lane group each), and a merge
+// sums each class's slice partials, a workgroup per class and 32 columns.
 #include "common.hpp"
 #include "gather.hpp"
 #include "slices.hpp"
@@ -256,11 +256,21 @@ int32_t mantis_class_reduce(const void* values, int32_t values_dtype, int64_t n_
   slice_edges_kernel<<<unsigned((L.n_slices + 1 + 255) / 256), 256, 0, s>>>(cls_ptr, slice_ptr, n_classes, n_entries,
                                                                              L.n_slices, slice_edge);
   if ((st = launched()) != MANTIS_OK) return st;
-  st = mantis_run_reduce(values, values_dtype, n_src, ld, h, gather, n_entries, slice_edge, L.n_slices, partial,
-                         MANTIS_F32, err_flag, stream);
+  if (h % 8 == 0 && ld % 8 == 0 && aligned16(values) && n_src <= 2147483647LL) {
+    const dim3 grid{unsigned((L.n_slices + 256 / kGroup - 1) / (256 / kGroup)),
+                    unsigned((h + kGroup * 8 - 1) / (kGroup * 8))};
+    const bool ok = with_type(values_dtype, [&](auto t) {
+      using T = decltype(t);
+      slice_sum_kernel<T><<<grid, 256, 0, s>>>(static_cast<const T*>(values), n_src, ld, h, gather, n_entries,
+                                               slice_edge, L.n_slices, partial, err_flag);
+    });
+    st = ok ? launched() : MANTIS_E_ARG;
+  } else {  // rows that 16-byte loads do not fit
+    st = mantis_run_reduce(values, values_dtype, n_src, ld, h, gather, n_entries, slice_edge, L.n_slices, partial,
+                           MANTIS_F32, err_flag, stream);
+  }
   if (st != MANTIS_OK) return st;
-  return mantis_run_reduce(partial, MANTIS_F32, L.n_slices, h, h, nullptr, L.n_slices, slice_ptr, n_classes, out,
-                           out_dtype, err_flag, stream);
+  return slice_merge(partial, h, slice_ptr, L.n_slices, n_classes, out, out_dtype, s);
 }
 
 int64_t mantis_cell_pass_backward_workspace(int64_t n_relay, int64_t n_edges, int64_t n_classes, int64_t h) {

@@ -1,18 +1,23 @@
 // Sliced reductions over unbounded runs (class-major entry lists, where one
 // class can own most of the entries): every run is cut into slices of at
 // most kSlice entries, each slice is summed into a partial row by its own
-// lane group, and a second run reduction sums each run's partials in slice
-// order.  The slice tables come from two small kernels: an exclusive scan of
-// the slice counts (slice_ptr, one per run) and the first entry of every
-// slice (slice_edge).  Deterministic: fixed slice bounds, fixed orders.
+// lane group, and slice_merge_kernel sums each run's partials, a workgroup
+// per run and 32 columns.  The slice tables come from two small kernels: an
+// exclusive scan of the slice counts (slice_ptr, one per run) and the first
+// entry of every slice (slice_edge).  Deterministic: fixed slice bounds,
+// fixed orders.
 #pragma once
 
 #include "common.hpp"
+#include "gather.hpp"
 
 namespace mantis {
 namespace {
 
-constexpr int64_t kSlice = 64;  // run entries per partial row
+// Run entries per partial row: the longest chain of a lane group (and of fp32
+// additions: at 128 the sums of 1,200 entries were 1.6 times as far from
+// float64), against the partial rows that the merge reads back.
+constexpr int64_t kSlice = 64;
 
 // slice_ptr[k] = first slice of class k: the exclusive prefix sum of
 // ceil(len_k / kSlice) over the classes (one workgroup, chunks of 1024).
@@ -74,6 +79,105 @@ __global__ void slice_edges_kernel(const int64_t* __restrict__ cls_ptr, const in
   int64_t a, b;
   segment(cls_ptr, lo, n_edges, a, b);
   slice_edge[s] = a + (s - slice_ptr[lo]) * kSlice;
+}
+
+// partial[s] = sum of values[gather[j]] over the entries j of slice s, columns
+// 128 blockIdx.y .. (16 lanes per slice and chunk, h a multiple of 8): 16
+// indices per load, kLook rows in flight.  Bound by the gathered rows.
+template <typename Tin>
+__global__ void __launch_bounds__(256)
+slice_sum_kernel(const Tin* __restrict__ values, int64_t n_src, int64_t ld, int64_t h,
+                 const int64_t* __restrict__ gather, int64_t n_entries, const int64_t* __restrict__ slice_edge,
+                 int64_t n_slices, float* __restrict__ partial, int32_t* flag) {
+  constexpr int kLook = 4;
+  const int64_t s = int64_t(blockIdx.x) * (256 / kGroup) + threadIdx.x / kGroup;
+  const int lane = threadIdx.x % kGroup;
+  if (s >= n_slices) return;
+  const int64_t c0 = int64_t(blockIdx.y) * (kGroup * 8) + lane * 8;
+  const bool mine = c0 < h;  // a lane past the width only shares its index
+  int64_t st, en;
+  segment(slice_edge, s, n_entries, st, en);
+  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int64_t base = st; base < en; base += kGroup) {
+    const int cnt = int(en - base < kGroup ? en - base : kGroup);
+    const int64_t g = gather[base + (lane < cnt ? lane : cnt - 1)];
+    const bool in = g >= 0 && g < n_src;
+    if (lane < cnt && !in) raise_flag(flag, MANTIS_FLAG_INDEX);
+    const int32_t row = in ? int32_t(g) : -1;  // n_src fits int32 (host check)
+    for (int j = 0; j < cnt; j += kLook) {
+      float x[kLook][8];
+      bool ok[kLook];
+#pragma unroll
+      for (int u = 0; u < kLook; ++u) {
+        const int32_t r = __shfl(row, j + u < cnt ? j + u : cnt - 1, kGroup);
+        ok[u] = mine && j + u < cnt && r >= 0;
+        if (ok[u]) load8(values + int64_t(r) * ld + c0, x[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kLook; ++u)
+        if (ok[u])
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i] += x[u][i];
+    }
+  }
+  if (mine) store8(partial + s * h + c0, acc);
+}
+
+// out[k] = sum of the partial rows of run k (slice_ptr[k] .. slice_ptr[k+1]),
+// one workgroup per run and 32 columns: 8 row groups, 8 rows in flight each,
+// then the groups by halves.  (A run of 10^5 entries has about 10^3 partial
+// rows; summed one after another by one lane group they were 170 us of every
+// class gradient at 64-96 positions, here under 20.)
+constexpr int kMergeCols = 32;
+template <typename To>
+__global__ void __launch_bounds__(256)
+slice_merge_kernel(const float* __restrict__ partial, int64_t h, const int64_t* __restrict__ slice_ptr,
+                   int64_t n_slices, To* __restrict__ out) {
+  constexpr int kGroups = 256 / kMergeCols;
+  __shared__ float red[kGroups][kMergeCols];
+  const int col = threadIdx.x % kMergeCols, g = threadIdx.x / kMergeCols;
+  const int64_t k = blockIdx.x, c = int64_t(blockIdx.y) * kMergeCols + col;
+  int64_t st, en;
+  segment(slice_ptr, k, n_slices, st, en);
+  float acc = 0.f;
+  if (c < h) {
+    for (int64_t s = st + g; s < en; s += 8 * kGroups) {
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int64_t r = s + u * kGroups;
+        x[u] = partial[(r < en ? r : s) * h + c];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += s + u * kGroups < en ? x[u] : 0.f;
+    }
+  }
+  red[g][col] = acc;
+  __syncthreads();
+#pragma unroll
+  for (int o = kGroups / 2; o > 0; o >>= 1) {
+    if (g < o) red[g][col] += red[g + o][col];
+    __syncthreads();
+  }
+  if (g == 0 && c < h) from_f32(out[k * h + c], red[0][col]);
+}
+
+template <typename To>
+int32_t slice_merge(const float* partial, int64_t h, const int64_t* slice_ptr, int64_t n_slices, int64_t n_runs,
+                    To* out, hipStream_t s) {
+  const dim3 grid{unsigned(n_runs), unsigned((h + kMergeCols - 1) / kMergeCols)};
+  slice_merge_kernel<To><<<grid, 256, 0, s>>>(partial, h, slice_ptr, n_slices, out);
+  return launched();
+}
+
+inline int32_t slice_merge(const float* partial, int64_t h, const int64_t* slice_ptr, int64_t n_slices,
+                           int64_t n_runs, void* out, int32_t out_dtype, hipStream_t s) {
+  switch (out_dtype) {
+    case MANTIS_F32: return slice_merge(partial, h, slice_ptr, n_slices, n_runs, static_cast<float*>(out), s);
+    case MANTIS_BF16: return slice_merge(partial, h, slice_ptr, n_slices, n_runs, static_cast<uint16_t*>(out), s);
+    case MANTIS_F16: return slice_merge(partial, h, slice_ptr, n_slices, n_runs, static_cast<_Float16*>(out), s);
+    default: return MANTIS_E_ARG;
+  }
 }
 
 inline int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }

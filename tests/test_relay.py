@@ -253,6 +253,34 @@ def test_class_reduce_spreads_a_dominant_class(device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("h,dt", [(8, torch.float32), (20, torch.float32), (128, torch.bfloat16),
+                                  (136, torch.float16), (512, torch.float32)])
+def test_class_reduce_run_lengths(device, h, dt):
+    """Runs around a slice (64 entries), around the merge's 8 row groups of 8
+    rows and past them, empty runs, and widths off the 32- and 128-column
+    chunks; an index out of range adds nothing and is flagged."""
+    gen = torch.Generator().manual_seed(14)
+    lens = torch.tensor([0, 1, 63, 64, 65, 511, 512, 513, 4096, 4161, 0, 9000])
+    cls_ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    values = torch.randn(300, h, generator=gen).to(dt)
+    rows = torch.randint(0, 300, (int(lens.sum()),), generator=gen)
+    cls = torch.repeat_interleave(torch.arange(len(lens)), lens)
+    ref = torch.zeros(len(lens), h, dtype=torch.float64).index_add_(0, cls, values.double()[rows])
+    got = mantisnet.ops.class_reduce(values.to(device), rows.to(device), cls_ptr.to(device), len(lens), torch.float32)
+    mantisnet.ops.raise_on_device_error(device)
+    # fp32 sums of n values near 1: 64 in a row, then a tree of partial sums
+    torch.testing.assert_close(got.double().cpu(), ref, rtol=1e-5, atol=1e-3)
+    rows[5], rows[-1] = 300, -1
+    keep = torch.ones(len(rows), dtype=torch.bool)
+    keep[5] = keep[-1] = False
+    ref = torch.zeros(len(lens), h, dtype=torch.float64).index_add_(0, cls[keep], values.double()[rows[keep]])
+    got = mantisnet.ops.class_reduce(values.to(device), rows.to(device), cls_ptr.to(device), len(lens), torch.float32)
+    torch.testing.assert_close(got.double().cpu(), ref, rtol=1e-5, atol=1e-3)
+    with pytest.raises(ValueError):
+        mantisnet.ops.raise_on_device_error(device)
+
+
+@pytest.mark.gpu
 def test_message_passing_backward_matches_autograd(device):
     batch = _batch(6, config=4, start=9)
     run_stone, run_window, run_class = R.incidence_plan(batch.inc_stone, batch.inc_window, batch.inc_class)
