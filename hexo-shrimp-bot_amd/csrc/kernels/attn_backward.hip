@@ -10,7 +10,7 @@
 //    the gradients are dq = scale sum_e dscore_e k[src_e],
 //    dk = scale sum_e dscore_e q[qid_e], dv = sum_e alpha_e go[qid_e],
 //    dbias[cls] = sum_e dscore_e and dvcls[cls] = sum_e alpha_e go[qid_e].
-//    A query-major pass forms delta, dq and the per-edge (alpha, dscore); a
+//    A query-major pass forms delta, dq and the per-edge (alpha, dalpha); a
 //    source-major pass recomputes each edge's score for dk and dv; the class
 //    sums are sliced reductions over the class-major edge list.
 //  * the action-row encoder (row_encoder.py:115-413): with
@@ -19,11 +19,14 @@
 //    dtable[c] = sum_e mask_e go[cell_e] over the class's entries.
 //
 // Geometry: 16 lanes per row of 4 heads x 32 (a lane owns 8 consecutive
-// features, a head is 4 adjacent lanes), entries walked one at a time, every
-// sum in fp32 in a fixed order: no atomics, and two calls agree bitwise.
+// features, a head is 4 adjacent lanes), the entries of a row loaded 16 at a
+// time, every sum in fp32 in a fixed order: no atomics, and two calls agree
+// bitwise.
 #include "common.hpp"
 #include "gather.hpp"
 #include "slices.hpp"
+
+#include <type_traits>
 
 namespace mantis {
 namespace {
@@ -53,69 +56,91 @@ struct AttnBwd {
   int32_t* flag;
 };
 
-__device__ __forceinline__ float expf_acc(float x) { return expf(x); }
-
-// the 8 features of a lane, as fp32
-template <typename T>
-__device__ __forceinline__ void row8(const void* base, int64_t row, int64_t ld, int64_t c0, float (&x)[8]) {
-  load8(static_cast<const T*>(base) + row * ld + c0, x);
-}
-
-template <typename T, typename Tv>
+// Query-major pass: 16 lanes per query row; up to 16 of its entries are loaded
+// at once, one per lane, and shared by shuffles, so the rows of kB entries are
+// in flight together (an entry at a time, each waited for its own chain of
+// index and rows).  Bound by the gathered rows.  With alpha_e, alpha and
+// dalpha of every entry are kept for the class sums; with finish the lane that
+// wrote them turns dalpha into dscore (callers without qid, whose class pass
+// cannot look delta up).
+template <typename T, typename Tv, bool kVcls>
 __global__ void __launch_bounds__(kBlock)
 attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t* __restrict__ src,
                   const int64_t* __restrict__ cls, int64_t n_entries, T* __restrict__ dq,
-                  float* __restrict__ alpha_e, float* __restrict__ dscore_e) {
+                  float* __restrict__ alpha_e, float* __restrict__ dalpha_e, bool finish) {
+  constexpr int kB = sizeof(T) == 2 ? 4 : 2;
   const int64_t row = int64_t(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
   const int lane = threadIdx.x % kGroup;
   if (row >= a.n_q) return;
   const int h = lane >> 2;
   const int64_t c0 = 8 * lane;
+  const T* kb = static_cast<const T*>(a.k) + c0;
+  const T* vb = static_cast<const T*>(a.v) + c0;
+  const Tv* cb = static_cast<const Tv*>(a.vcls) + c0;
+  int64_t st, en;
+  segment(seg_ptr, row, n_entries, st, en);
   float qv[8], gv[8];
-  row8<T>(a.q, row, a.ldq, c0, qv);
+  load8(static_cast<const T*>(a.q) + row * a.ldq + c0, qv);
   load8(a.go + row * a.ldgo + c0, gv);
   const float mm = a.m[row * kHeads + h], ll = a.l[row * kHeads + h];
   const float inv = ll > 0.f ? 1.f / ll : 0.f;
-  int64_t st, en;
-  segment(seg_ptr, row, n_entries, st, en);
   float A[8] = {0, 0, 0, 0, 0, 0, 0, 0}, B[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   float delta = 0.f;
-  for (int64_t e = st; e < en; ++e) {
-    const int64_t s = src[e], c = cls ? cls[e] : 0;
-    const bool ok = s >= 0 && s < a.n_k && c >= 0 && (!cls || c < a.n_classes);
-    if (!ok) {  // uniform over the group: every lane reads the same entry
-      if (lane == 0) raise_flag(a.flag, MANTIS_FLAG_INDEX);
-      if (alpha_e && (lane & 3) == 0) alpha_e[e * kHeads + h] = dscore_e[e * kHeads + h] = 0.f;
-      continue;
-    }
-    float kv[8], vv[8];
-    row8<T>(a.k, s, a.ldk, c0, kv);
-    row8<T>(a.v, s, a.ldv, c0, vv);
-    if (a.vcls) {
-      float cv[8];
-      row8<Tv>(a.vcls, c, kRow, c0, cv);
+  for (int64_t base = st; base < en; base += kGroup) {
+    const int cnt = int(en - base < kGroup ? en - base : kGroup);
+    const int64_t mine = base + (lane < cnt ? lane : cnt - 1);
+    const int64_t s = src[mine], c = cls ? cls[mine] : 0;
+    const bool good = s >= 0 && s < a.n_k && c >= 0 && (!cls || c < a.n_classes);
+    if (!good && lane < cnt) raise_flag(a.flag, MANTIS_FLAG_INDEX);
+    const int64_t s_ok = good ? s : 0;
+    const int32_t c_ok = good ? int32_t(c) : 0;
+    for (int j = 0; j < cnt; j += kB) {
+      Chunk8<T> xk[kB], xv[kB];
+      Chunk8<Tv> xc[kB];
+      float bs[kB];
+      bool ok[kB];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) vv[i] += cv[i];
-    }
-    float sd = 0.f, dd = 0.f;
+      for (int u = 0; u < kB; ++u) {
+        const int from = j + u < cnt ? j + u : cnt - 1;
+        const int64_t su = __shfl(s_ok, from, kGroup);
+        const int32_t cu = __shfl(c_ok, from, kGroup);
+        ok[u] = __shfl(int(good), from, kGroup) != 0 && j + u < cnt;
+        if (a.n_k > 0) {  // (an entry that is not ok reads row 0)
+          xk[u].load(kb + su * a.ldk);
+          xv[u].load(vb + su * a.ldv);
+        }
+        if constexpr (kVcls) xc[u].load(cb + int64_t(cu) * kRow);
+        bs[u] = a.bias ? a.bias[h * a.n_classes + cu] : 0.f;
+      }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      sd = fmaf(qv[i], kv[i], sd);
-      dd = fmaf(gv[i], vv[i], dd);
-    }
-    sd = head_sum(sd);
-    dd = head_sum(dd);
-    const float score = sd * a.scale + (a.bias ? a.bias[h * a.n_classes + c] : 0.f);
-    const float al = expf_acc(score - mm) * inv;
-    delta = fmaf(al, dd, delta);
+      for (int u = 0; u < kB; ++u) {
+        const int64_t e = base + j + u;
+        if (!ok[u]) {  // uniform over the group
+          if (j + u < cnt && alpha_e && (lane & 3) == 0) alpha_e[e * kHeads + h] = dalpha_e[e * kHeads + h] = 0.f;
+          continue;
+        }
+        float sd = 0.f, dd = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      A[i] = fmaf(al * dd, kv[i], A[i]);
-      B[i] = fmaf(al, kv[i], B[i]);
-    }
-    if (alpha_e && (lane & 3) == 0) {
-      alpha_e[e * kHeads + h] = al;
-      dscore_e[e * kHeads + h] = dd;  // dalpha for now; dscore below, once delta is known
+        for (int i = 0; i < 8; ++i) {
+          float vv = xv[u][i];
+          if constexpr (kVcls) vv += xc[u][i];
+          sd = fmaf(qv[i], xk[u][i], sd);
+          dd = fmaf(gv[i], vv, dd);
+        }
+        sd = head_sum(sd);
+        dd = head_sum(dd);
+        const float al = expf(sd * a.scale + bs[u] - mm) * inv;
+        delta = fmaf(al, dd, delta);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          A[i] = fmaf(al * dd, xk[u][i], A[i]);
+          B[i] = fmaf(al, xk[u][i], B[i]);
+        }
+        if (alpha_e && (lane & 3) == 0) {
+          alpha_e[e * kHeads + h] = al;
+          dalpha_e[e * kHeads + h] = dd;
+        }
+      }
     }
   }
   float d[8];
@@ -125,76 +150,130 @@ attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t*
   if ((lane & 3) == 0) {
     a.delta[row * kHeads + h] = delta;
     // this lane wrote these entries above: dscore = alpha (dalpha - delta)
-    if (alpha_e)
+    if (finish)
       for (int64_t e = st; e < en; ++e)
-        dscore_e[e * kHeads + h] = alpha_e[e * kHeads + h] * (dscore_e[e * kHeads + h] - delta);
+        dalpha_e[e * kHeads + h] = alpha_e[e * kHeads + h] * (dalpha_e[e * kHeads + h] - delta);
   }
 }
 
-template <typename T, typename Tv>
+// Source-major pass: kG lane groups per source row, each taking every kG-th
+// chunk of 16 entries, their sums added in group order.  One group for short
+// runs (windows and cells: about five entries); a stone's run of 200 radius
+// entries left 5,000 groups each walking its own chain, a quarter of a
+// launch's lanes, so long runs get 4 groups (a wavefront) or 16 (a workgroup).
+template <typename T, typename Tv, bool kVcls, int kG>
 __global__ void __launch_bounds__(kBlock)
 attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_t* __restrict__ sqid,
                    const int64_t* __restrict__ scls, int64_t n_entries, T* __restrict__ dk, T* __restrict__ dv) {
-  const int64_t row = int64_t(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
+  static_assert(kG == 1 || kG == 4 || kG == kGroupsPerBlock);
+  constexpr int kB = 2;
+  const int group = threadIdx.x / kGroup;
+  const int64_t row = int64_t(blockIdx.x) * (kGroupsPerBlock / kG) + group / kG;
   const int lane = threadIdx.x % kGroup;
-  if (row >= a.n_k) return;
+  if (row >= a.n_k) return;  // uniform over the groups of a row
   const int h = lane >> 2;
   const int64_t c0 = 8 * lane;
-  float kv[8], vv[8];
-  row8<T>(a.k, row, a.ldk, c0, kv);
-  row8<T>(a.v, row, a.ldv, c0, vv);
+  const T* qb = static_cast<const T*>(a.q) + c0;
+  const float* gb = a.go + c0;
+  const Tv* cb = static_cast<const Tv*>(a.vcls) + c0;
   int64_t st, en;
   segment(sseg_ptr, row, n_entries, st, en);
+  float kv[8], vv[8];
+  load8(static_cast<const T*>(a.k) + row * a.ldk + c0, kv);
+  load8(static_cast<const T*>(a.v) + row * a.ldv + c0, vv);
   float gk[8] = {0, 0, 0, 0, 0, 0, 0, 0}, gvv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int64_t e = st; e < en; ++e) {
-    const int64_t qi = sqid[e], c = scls ? scls[e] : 0;
-    const bool ok = qi >= 0 && qi < a.n_q && c >= 0 && (!scls || c < a.n_classes);
-    if (!ok) {
-      if (lane == 0) raise_flag(a.flag, MANTIS_FLAG_INDEX);
-      continue;
-    }
-    float qv[8], gv[8], ve[8];
-    row8<T>(a.q, qi, a.ldq, c0, qv);
-    load8(a.go + qi * a.ldgo + c0, gv);
+  for (int64_t base = st + int64_t(group % kG) * kGroup; base < en; base += kG * kGroup) {
+    const int cnt = int(en - base < kGroup ? en - base : kGroup);
+    const int64_t mine = base + (lane < cnt ? lane : cnt - 1);
+    const int64_t qi = sqid[mine], c = scls ? scls[mine] : 0;
+    const bool good = qi >= 0 && qi < a.n_q && c >= 0 && (!scls || c < a.n_classes);
+    if (!good && lane < cnt) raise_flag(a.flag, MANTIS_FLAG_INDEX);
+    const int64_t q_ok = good ? qi : 0;
+    const int32_t c_ok = good ? int32_t(c) : 0;
+    for (int j = 0; j < cnt; j += kB) {
+      Chunk8<T> xq[kB];
+      Chunk8<float> xg[kB];
+      Chunk8<Tv> xc[kB];
+      float bs[kB], ml[kB], ll[kB], dl[kB];
+      bool ok[kB];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ve[i] = vv[i];
-    if (a.vcls) {
-      float cv[8];
-      row8<Tv>(a.vcls, c, kRow, c0, cv);
+      for (int u = 0; u < kB; ++u) {
+        const int from = j + u < cnt ? j + u : cnt - 1;
+        const int64_t qu = __shfl(q_ok, from, kGroup);
+        const int32_t cu = __shfl(c_ok, from, kGroup);
+        ok[u] = __shfl(int(good), from, kGroup) != 0 && j + u < cnt;
+        if (a.n_q > 0) {  // (an entry that is not ok reads row 0)
+          xq[u].load(qb + qu * a.ldq);
+          xg[u].load(gb + qu * a.ldgo);
+          ml[u] = a.m[qu * kHeads + h];
+          ll[u] = a.l[qu * kHeads + h];
+          dl[u] = a.delta[qu * kHeads + h];
+        }
+        if constexpr (kVcls) xc[u].load(cb + int64_t(cu) * kRow);
+        bs[u] = a.bias ? a.bias[h * a.n_classes + cu] : 0.f;
+      }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) ve[i] += cv[i];
-    }
-    float sd = 0.f, dd = 0.f;
+      for (int u = 0; u < kB; ++u) {
+        if (!ok[u]) continue;  // uniform over the group
+        float sd = 0.f, dd = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      sd = fmaf(qv[i], kv[i], sd);
-      dd = fmaf(gv[i], ve[i], dd);
-    }
-    sd = head_sum(sd);
-    dd = head_sum(dd);
-    const float score = sd * a.scale + (a.bias ? a.bias[h * a.n_classes + c] : 0.f);
-    const float ll = a.l[qi * kHeads + h];
-    const float al = ll > 0.f ? expf_acc(score - a.m[qi * kHeads + h]) / ll : 0.f;
-    const float ds = al * (dd - a.delta[qi * kHeads + h]);
+        for (int i = 0; i < 8; ++i) {
+          float ve = vv[i];
+          if constexpr (kVcls) ve += xc[u][i];
+          sd = fmaf(xq[u][i], kv[i], sd);
+          dd = fmaf(xg[u][i], ve, dd);
+        }
+        sd = head_sum(sd);
+        dd = head_sum(dd);
+        const float al = ll[u] > 0.f ? expf(sd * a.scale + bs[u] - ml[u]) / ll[u] : 0.f;
+        const float ds = al * (dd - dl[u]);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      gk[i] = fmaf(ds * a.scale, qv[i], gk[i]);
-      gvv[i] = fmaf(al, gv[i], gvv[i]);
+        for (int i = 0; i < 8; ++i) {
+          gk[i] = fmaf(ds * a.scale, xq[u][i], gk[i]);
+          gvv[i] = fmaf(al, xg[u][i], gvv[i]);
+        }
+      }
     }
   }
-  store8(dk + row * kRow + c0, gk);
-  store8(dv + row * kRow + c0, gvv);
+  if constexpr (kG > 1) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      gk[i] = sum_xor32(sum_xor16(gk[i]));
+      gvv[i] = sum_xor32(sum_xor16(gvv[i]));
+    }
+  }
+  if constexpr (kG == kGroupsPerBlock) {  // one row per workgroup: the wavefronts in order
+    __shared__ float red[kBlock / 64][2][kRow];
+    if ((threadIdx.x & 63) < kGroup)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        red[threadIdx.x / 64][0][c0 + i] = gk[i];
+        red[threadIdx.x / 64][1][c0 + i] = gvv[i];
+      }
+    __syncthreads();
+    if (threadIdx.x < kGroup)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        gk[i] = ((red[0][0][c0 + i] + red[1][0][c0 + i]) + red[2][0][c0 + i]) + red[3][0][c0 + i];
+        gvv[i] = ((red[0][1][c0 + i] + red[1][1][c0 + i]) + red[2][1][c0 + i]) + red[3][1][c0 + i];
+      }
+  }
+  if (group % kG == 0) {
+    store8(dk + row * kRow + c0, gk);
+    store8(dv + row * kRow + c0, gvv);
+  }
 }
 
 // Class slices: partial4[s] = sum over the class-major entries j of slice s of
 // dscore[E], E = cedge[j] (a query-major edge), and with kV partial[s] = sum
-// of alpha[E, head] * go[qid[E]].  16 entries per index load; the gradient
+// of alpha[E, head] * go[qid[E]].  dscore = alpha (dalpha - delta[qid]), or
+// with qid null dalpha_e already holds it.  16 entries per index load; the gradient
 // rows of kLook entries in flight, the scores one entry per lane.  Bound by
 // the gathered gradient rows.
 template <bool kV>
 __global__ void __launch_bounds__(kBlock)
-class_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ dscore_e,
-                   const float* __restrict__ go, int64_t ldgo, const int64_t* __restrict__ qid, int64_t n_q,
+class_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ dalpha_e,
+                   const float* __restrict__ delta, const float* __restrict__ go, int64_t ldgo, const int64_t* __restrict__ qid, int64_t n_q,
                    const int64_t* __restrict__ cedge, int64_t n_edges, const int64_t* __restrict__ slice_edge,
                    int64_t n_slices, float* __restrict__ partial, float* __restrict__ partial4, int32_t* flag) {
   constexpr int kLook = 4;
@@ -212,15 +291,21 @@ class_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ 
     const int64_t E = cedge[base + (lane < cnt ? lane : cnt - 1)];
     bool ok = E >= 0 && E < n_edges;
     int64_t qi = 0;
-    if (ok && lane < cnt) {
-      const float4 d = *reinterpret_cast<const float4*>(dscore_e + E * kHeads);
-      d4.x += d.x, d4.y += d.y, d4.z += d.z, d4.w += d.w;
-    }
-    if constexpr (kV) {
+    if (qid) {
       qi = ok ? qid[E] : -1;
       ok = qi >= 0 && qi < n_q;
     }
     if (!ok && lane < cnt) raise_flag(flag, MANTIS_FLAG_INDEX);
+    if (ok && lane < cnt) {
+      float4 d = *reinterpret_cast<const float4*>(dalpha_e + E * kHeads);
+      if (qid) {
+        const float4 al = *reinterpret_cast<const float4*>(alpha_e + E * kHeads);
+        const float4 dl = *reinterpret_cast<const float4*>(delta + qi * kHeads);
+        d.x = al.x * (d.x - dl.x), d.y = al.y * (d.y - dl.y);
+        d.z = al.z * (d.z - dl.z), d.w = al.w * (d.w - dl.w);
+      }
+      d4.x += d.x, d4.y += d.y, d4.z += d.z, d4.w += d.w;
+    }
     if constexpr (kV) {
       const int64_t row = ok ? qi : -1;
       for (int j = 0; j < cnt; j += kLook) {
@@ -310,10 +395,10 @@ bool with_type(int32_t dtype, F&& fn) {
   }
 }
 
-// Workspace of the attention backward: delta, per-edge alpha and dscore,
+// Workspace of the attention backward: delta, per-edge alpha and dalpha,
 // the class slice tables and the two kinds of partial rows.
 struct AttnLayout {
-  int64_t delta, alpha, dscore, slices, total;
+  int64_t delta, alpha, dalpha, slices, total;
 };
 
 // (untyped edges, n_classes == 0, need delta alone)
@@ -322,11 +407,11 @@ AttnLayout attn_layout(int64_t n_q, int64_t n_edges, int64_t n_classes) {
   L.delta = 0;
   L.alpha = L.delta + align256(n_q * kHeads * 4);
   if (n_classes == 0) {
-    L.dscore = L.slices = L.total = L.alpha;
+    L.dalpha = L.slices = L.total = L.alpha;
     return L;
   }
-  L.dscore = L.alpha + align256(n_edges * kHeads * 4);
-  L.slices = L.dscore + align256(n_edges * kHeads * 4);
+  L.dalpha = L.alpha + align256(n_edges * kHeads * 4);
+  L.slices = L.dalpha + align256(n_edges * kHeads * 4);
   // slice tables + 128-wide partials, then 4-wide partials
   const SliceLayout S = slice_layout(n_edges, n_classes, kRow);
   L.total = L.slices + S.total + align256(S.n_slices * kHeads * 4);
@@ -375,20 +460,32 @@ int32_t mantis_attention_backward(const void* q, const void* k, const void* v, i
             reinterpret_cast<float*>(ws + L.delta), 0.17677669529663687f, err_flag};
   // per-edge softmax terms: kept for the class sums of typed edges only
   float* alpha_e = typed ? reinterpret_cast<float*>(ws + L.alpha) : nullptr;
-  float* dscore_e = typed ? reinterpret_cast<float*>(ws + L.dscore) : nullptr;
+  float* dalpha_e = typed ? reinterpret_cast<float*>(ws + L.dalpha) : nullptr;
   hipStream_t s = as_stream(stream);
   bool ok_v = true;
   const bool ok = with_type(dtype, [&](auto t) {
     using T = decltype(t);
     auto run = [&](auto tv) {
       using Tv = decltype(tv);
-      if (n_q > 0)
-        attn_bwd_q_kernel<T, Tv><<<grid_rows(n_q), kBlock, 0, s>>>(a, seg_ptr, src, typed ? cls : nullptr, n_entries,
-                                                                    static_cast<T*>(dq), alpha_e, dscore_e);
-      if (n_k > 0)
-        attn_bwd_kv_kernel<T, Tv><<<grid_rows(n_k), kBlock, 0, s>>>(a, sseg_ptr, sqid, typed ? scls : nullptr,
-                                                                     n_entries, static_cast<T*>(dk),
-                                                                     static_cast<T*>(dv));
+      auto passes = [&](auto with_vcls) {
+        constexpr bool kV = decltype(with_vcls)::value;
+        if (n_q > 0)
+          attn_bwd_q_kernel<T, Tv, kV><<<grid_rows(n_q), kBlock, 0, s>>>(
+              a, seg_ptr, src, typed ? cls : nullptr, n_entries, static_cast<T*>(dq), alpha_e, dalpha_e,
+              typed && !qid);
+        if (n_k == 0) return;
+        auto kv = [&](auto groups) {
+          constexpr int kG = decltype(groups)::value;
+          attn_bwd_kv_kernel<T, Tv, kV, kG><<<grid_rows(n_k * kG), kBlock, 0, s>>>(
+              a, sseg_ptr, sqid, typed ? scls : nullptr, n_entries, static_cast<T*>(dk), static_cast<T*>(dv));
+        };
+        // a mean run of one chunk of 16 entries per group of the row
+        if (n_entries < 16 * n_k) kv(std::integral_constant<int, 1>{});
+        else if (n_entries < 64 * n_k) kv(std::integral_constant<int, 4>{});
+        else kv(std::integral_constant<int, kGroupsPerBlock>{});
+      };
+      if (vcls) passes(std::true_type{});
+      else passes(std::false_type{});
     };
     if (!vcls) run(float{});
     else ok_v = with_type(vcls_dtype, run);
@@ -410,7 +507,7 @@ int32_t mantis_attention_backward(const void* q, const void* k, const void* v, i
                                                                              S.n_slices, slice_edge);
   if ((st = launched()) != MANTIS_OK) return st;
   auto slices = vcls ? class_slice_kernel<true> : class_slice_kernel<false>;
-  slices<<<grid_rows(S.n_slices), kBlock, 0, s>>>(alpha_e, dscore_e, grad_out, ldgo, qid, n_q, cedge_q, n_entries,
+  slices<<<grid_rows(S.n_slices), kBlock, 0, s>>>(alpha_e, dalpha_e, a.delta, grad_out, ldgo, qid, n_q, cedge_q, n_entries,
                                                   slice_edge, S.n_slices, partial, partial4, err_flag);
   if ((st = launched()) != MANTIS_OK) return st;
   st = slice_merge(partial4, kHeads, slice_ptr, S.n_slices, n_classes, dbias_t, s);

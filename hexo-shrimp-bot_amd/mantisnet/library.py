@@ -356,17 +356,28 @@ def _(q, k, v, bias, seg_ptr, src, cls, qid, sseg_ptr, sqid, scls, cptr, cedge_q
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty_like(bias)
 
 
+def _out_grad(grad_out, ctx) -> Tensor:
+    """The gradient of a segment attention's fp32 output, shaped like its
+    queries (zeros when only the statistics were differentiated)."""
+    q = ctx.saved_tensors[0]
+    return torch.zeros(q.shape, dtype=torch.float32, device=q.device) if grad_out is None else grad_out
+
+
 def _ca_setup(ctx, inputs, output) -> None:
     _out, m, l = output
     ctx.save_for_backward(*inputs, m, l)
+    # the statistics' gradients are not used: no zero tensors made for them
+    ctx.set_materialize_grads(False)
 
 
 def _ca_backward(ctx, grad_out, _gm, _gl):
+    grad_out = _out_grad(grad_out, ctx)
     grads = cell_attention_backward(*ctx.saved_tensors, grad_out)
     return grads + (None,) * 9
 
 
 def _ca_plain_backward(ctx, grad_out, _gm, _gl):
+    grad_out = _out_grad(grad_out, ctx)
     grads = cell_attention_plain_backward(*ctx.saved_tensors, grad_out)
     return grads + (None,) * 9
 
@@ -456,9 +467,11 @@ def _(q, k, v, window_pos, offsets, order, m, l, grad_out):
 def _read_setup(ctx, inputs, output) -> None:
     out, m, l = output
     ctx.save_for_backward(*inputs, out, m, l)
+    ctx.set_materialize_grads(False)
 
 
 def _read_backward(ctx, grad_out, _gm, _gl):
+    grad_out = _out_grad(grad_out, ctx)
     dq, dk, dv = window_latent_read_backward(*ctx.saved_tensors, grad_out)
     return dq, dk, dv, None, None, None
 
@@ -466,9 +479,11 @@ def _read_backward(ctx, grad_out, _gm, _gl):
 def _broadcast_setup(ctx, inputs, output) -> None:
     _out, m, l = output
     ctx.save_for_backward(*inputs, m, l)
+    ctx.set_materialize_grads(False)
 
 
 def _broadcast_backward(ctx, grad_out, _gm, _gl):
+    grad_out = _out_grad(grad_out, ctx)
     dq, dk, dv = window_latent_broadcast_backward(*ctx.saved_tensors, grad_out)
     return dq, dk, dv, None, None, None
 

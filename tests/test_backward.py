@@ -108,6 +108,36 @@ def test_window_latent_backward(device, batch):
     mantisnet.ops.raise_on_device_error(device)
 
 
+@pytest.mark.parametrize("n_k,dt,with_vcls", [(400, torch.float32, True), (19, torch.float32, False),
+                                              (18, torch.float16, True), (5, torch.float32, True),
+                                              (4, torch.bfloat16, False), (1, torch.float32, True)])
+def test_cell_attention_backward_run_lengths(device, n_k, dt, with_vcls):
+    """300 entries over few or many source rows: mean source runs either side
+    of 16 and 64 entries (one, 4 or 16 lane groups per row), query runs of 0
+    to over 16 entries, one class owning most entries."""
+    gen = torch.Generator().manual_seed(27 + n_k)
+    n_q, n_e = 33, 300
+    dst = torch.cat([torch.full((40,), 7), torch.randint(8, n_q, (n_e - 40,), generator=gen)])
+    src = torch.randint(0, n_k, (n_e,), generator=gen)
+    cls = torch.where(torch.rand(n_e, generator=gen) < 0.7, 2, torch.randint(0, 5, (n_e,), generator=gen))
+    t = R.edge_tables_full(src, dst, cls, torch.zeros(0, dtype=torch.long), n_k, n_q, 5, False)
+    views = [t[n].to(device) for n in ("dst_ptr", "edge_src", "edge_class", "edge_dst", "source_ptr", "edge_sdst",
+                                       "edge_sclass", "cls_ptr", "cedge_dst")]
+    inputs = [torch.randn(n, 4, 32, generator=gen).to(dt) for n in (n_q, n_k, n_k)]
+    inputs += [0.3 * torch.randn(4, 5, generator=gen)] + ([0.1 * torch.randn(5, 128, generator=gen)] if with_vcls else [])
+    seed = torch.randn(n_q, 4, 32, generator=gen)
+    op = OPS.cell_attention if with_vcls else OPS.cell_attention_plain
+
+    def ref(q, k, v, b, c=None):
+        return R.cell_attention(q, k, v, b, c, t["edge_src"], t["edge_class"], t["edge_dst"])
+
+    got = _grads(lambda *x: op(*x, *views)[0], [x.to(device) for x in inputs], seed.to(device))
+    mantisnet.ops.raise_on_device_error(device)
+    _close(got, _grads(ref, [x.float() for x in inputs], seed), dt)
+    again = _grads(lambda *x: op(*x, *views)[0], [x.to(device) for x in inputs], seed.to(device))
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
 @pytest.mark.parametrize("counts,dt,shuffled", [
     ([0], torch.float32, False), ([1], torch.float32, False), ([63, 64, 65], torch.float32, True),
     ([3, 0, 700, 17], torch.float32, True), ([130, 1, 0], torch.bfloat16, False), ([16, 15, 257], torch.float16, True),
