@@ -49,6 +49,8 @@ SIGNATURES = {
     "mantis_attention_backward_workspace": ([i64, i64, i64], i64),
     "mantis_attention_backward": ([vp, vp, vp, i32, i64, i64, i64, i64, i64, vp, i64, vp, i32, vp, i64, vp, vp, vp,
                                    vp, vp, vp, i64, vp, vp, vp, vp, vp, vp, i64, vp, vp, vp, vp, vp, vp, vp], i32),
+    "mantis_class_order_workspace": ([i64, i64], i64),
+    "mantis_class_order": ([vp, vp, i64, i64, vp, vp, vp, i64, vp, vp], i32),
     "mantis_latent_backward_workspace": ([i64, i64], i64),
     "mantis_latent_read_backward": ([vp, vp, vp, i32, i64, i64, i64, vp, vp, vp, i64, i64, vp, vp, vp, vp, vp, i64, vp,
                                      vp, vp, vp, vp], i32),

@@ -186,9 +186,8 @@ def _class_row_sum_backward(ctx, grad_out):
     # (message_passing.py:380-397): the class-major view of the entries, then
     # the sliced class reduction
     gather, runs = ctx.saved_tensors
-    order = torch.argsort(gather, stable=True)
-    cls_ptr = ops.runs_to_ptr(gather.index_select(0, order), ctx.n_classes)
-    grad = ops.class_reduce(grad_out, runs.index_select(0, order), cls_ptr, ctx.n_classes, ctx.weight_dtype)
+    cls_ptr, rows = ops.class_order(gather, ctx.n_classes, runs)
+    grad = ops.class_reduce(grad_out, rows, cls_ptr, ctx.n_classes, ctx.weight_dtype)
     return grad, None, None, None, None
 
 

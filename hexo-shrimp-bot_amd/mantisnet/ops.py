@@ -568,6 +568,32 @@ def class_reduce(values: Tensor, gather: Tensor, cls_ptr: Tensor, n_classes: int
     return out
 
 
+CLASS_ORDER_KEYS = 2048  # the key counters of a wavefront in LDS
+
+
+def class_order(key: Tensor, n_keys: int, col: Tensor | None = None) -> tuple[Tensor, Tensor]:
+    """(ptr, entries): the CSR over the keys and the entries' indices (or
+    their ``col`` values) in stable key order, by a counting sort for up to
+    2,048 keys (every class vocabulary here) and by torch's sort past that."""
+    dev = _on_gpu(key, col)
+    key = _i64(key, "key")
+    col = None if col is None else _i64(col, "col")
+    n = key.numel()
+    if col is not None and col.numel() != n:
+        raise ValueError("key and col must have one length")
+    if not 0 < n_keys <= CLASS_ORDER_KEYS or n >= 2**31 - 1024:
+        order = torch.argsort(key, stable=True)
+        ptr = runs_to_ptr(key.index_select(0, order), n_keys)
+        return ptr, order if col is None else col.index_select(0, order)
+    ptr = torch.empty(n_keys + 1, dtype=torch.int64, device=dev)
+    out = torch.empty(n, dtype=torch.int64, device=dev)
+    ws = _workspace(_lib().mantis_class_order_workspace(n, n_keys), dev)
+    _launch("class_order", 8.0 * (2 * n + n_keys + (0 if col is None else n)), 0.0, lambda: _check(
+        _lib().mantis_class_order(_ptr(key), _ptr(col), n, n_keys, _ptr(ptr), _ptr(out), _ptr(ws), ws.numel(),
+                                  _ptr(error_flag(dev)), _stream()), "class_order"))
+    return ptr, out
+
+
 def _check_cell_pass(x, emb, cell_ptr, edge_window, edge_class, win_ptr, edge_wcell, cls_ptr=None,
                      edge_ccell=None) -> None:
     """The reference's argument checks (relay.py:268-289), before any device check."""
@@ -753,8 +779,7 @@ def row_encode_backward(pre: Tensor, table: Tensor, edge_window: Tensor, edge_cl
     n_w, n_cls, n_cells = pre.shape[0], table.shape[0], grad_out.shape[0]
     go = grad_out.reshape(n_cells, 128).float().contiguous()
     win_ptr = runs_to_ptr(edge_window.index_select(0, edge_rev), n_w)
-    cls_order = torch.argsort(edge_class, stable=True)
-    cls_ptr = runs_to_ptr(edge_class.index_select(0, cls_order), n_cls)
+    cls_ptr, cls_order = class_order(edge_class, n_cls)
     e = edge_window.numel()
     dpre = torch.empty((n_w, 128), dtype=pre.dtype, device=dev)
     dtable = torch.empty((n_cls, 128), dtype=table.dtype, device=dev)

@@ -273,6 +273,19 @@ int32_t mantis_attention_backward(const void* q, const void* k, const void* v, i
                                   void* dk, void* dv, float* dbias_t, void* dvcls, int32_t* err_flag, void* stream);
 
 /*
+ * The stable key-major order of an entry list with few keys (class ids,
+ * n_keys <= 2048): ptr (n_keys + 1) the CSR over keys, out the entry indices
+ * (or with col non-NULL col's values) in key order, ties in entry order.
+ * Entries with a key outside [0, n_keys) are flagged and left out.  workspace:
+ * mantis_class_order_workspace(n_entries, n_keys) bytes (-1: out of range),
+ * 16-byte aligned.  Replaces the argsorts of the class gradients
+ * (message_passing.py:380-397, row_encoder.py:300-413).
+ */
+int64_t mantis_class_order_workspace(int64_t n_entries, int64_t n_keys);
+int32_t mantis_class_order(const int64_t* key, const int64_t* col, int64_t n_entries, int64_t n_keys, int64_t* ptr,
+                           int64_t* out, void* workspace, int64_t workspace_bytes, int32_t* err_flag, void* stream);
+
+/*
  * Backward of the window-latent read (latent queries q (4 n_pos rows) over
  * window keys and values k, v (n_w rows)) and broadcast (window queries q
  * over latent keys and values), rows of 4 heads x 32 in dtype with strides

@@ -281,6 +281,28 @@ def test_class_reduce_run_lengths(device, h, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,n_keys", [(0, 5), (1, 1), (63, 2), (1024, 726), (1025, 729), (4097, 1458),
+                                      (70001, 2048), (3000, 2049)])
+def test_class_order(device, n, n_keys):
+    """Around the 1,024-entry tiles and the 2,048-key limit, one key owning
+    half the entries: the stable argsort and its CSR."""
+    gen = torch.Generator().manual_seed(15 + n)
+    key = torch.where(torch.rand(n, generator=gen) < 0.5, n_keys // 2, torch.randint(0, n_keys, (n,), generator=gen))
+    col = torch.randint(0, 10**12, (n,), generator=gen)
+    order = torch.argsort(key, stable=True)
+    ptr = torch.searchsorted(key[order].contiguous(), torch.arange(n_keys + 1))
+    for c, exp in ((None, order), (col, col[order])):
+        got = mantisnet.ops.class_order(key.to(device), n_keys, None if c is None else c.to(device))
+        assert torch.equal(got[0].cpu(), ptr) and torch.equal(got[1].cpu(), exp)
+    mantisnet.ops.raise_on_device_error(device)
+    if n:
+        key[n // 2] = n_keys
+        mantisnet.ops.class_order(key.to(device), n_keys)
+        with pytest.raises(ValueError):
+            mantisnet.ops.raise_on_device_error(device)
+
+
+@pytest.mark.gpu
 def test_message_passing_backward_matches_autograd(device):
     batch = _batch(6, config=4, start=9)
     run_stone, run_window, run_class = R.incidence_plan(batch.inc_stone, batch.inc_window, batch.inc_class)
