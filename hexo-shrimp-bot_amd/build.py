@@ -20,7 +20,7 @@ PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
-HIP_SOURCES = ["gather_ops.hip", "stone_attention.hip", "hex_message.hip", "fused_linear.hip", "heads.hip",
+HIP_SOURCES = ["gather_ops.hip", "stone_attention.hip", "stone_attention_backward.hip", "hex_message.hip", "fused_linear.hip", "heads.hip",
                "attention_substage.hip", "cell_heads.hip", "latent_mix.hip", "improve.hip", "relay.hip", "attn_backward.hip", "plan.hip", "latent_broadcast.hip",
                "latent_read.hip", "latent_backward.hip", "class_order.hip", "radius_stage.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -397,226 +397,6 @@ stone_attention_kernel(const uint16_t* __restrict__ q, int64_t qsp, int64_t qsa,
 // [0, 128), [128, 256) and [256, 384) of the projected rows (row p * T + t;
 // head a at 32 a).  One workgroup per position: 16 lanes per (head, query)
 // row, each over every 16th key, the scores of the position staged in LDS.
-// Backward of the ragged attention (the reference's flash backward,
-// attention.py:166-560, with its row statistic delta = sum(out * grad_out)).
-// With a_ij = exp(scale q_i . k_j - lse_i) over the live keys j < L of the
-// live rows i < L, dp_ij = go_i . v_j and ds_ij = a_ij (dp_ij - delta_i):
-//   dq_i = scale sum_j ds_ij k_j,  dk_j = scale sum_i ds_ij q_i,  dv_j = sum_i a_ij go_i.
-// Two passes, each with a row per lane (two adjacent lanes per row for
-// HD = 64, each holding half of its dims): the query-major pass forms delta
-// and dq over the position's keys, the key-major pass dk and dv over its
-// queries; the other side's rows are staged in LDS in 64-row chunks, as fp32.
-// Every sum is fp32 in a fixed order (no atomics): two calls agree bitwise.
-// Rows and keys at or past L get zero gradients.
-template <int HD>
-struct BwdGeom {
-  static constexpr int kSplit = HD == 64 ? 2 : 1;  // lanes per row
-  static constexpr int kDims = HD / kSplit;         // dims per lane
-  static constexpr int kRows = 256 / kSplit;        // rows per workgroup
-};
-constexpr int kBwdChunk = 64;
-
-template <bool kHalf>
-__device__ __forceinline__ float bits_to_f32(uint16_t u) {
-  if constexpr (kHalf) return float(__builtin_bit_cast(_Float16, u));
-  else return bf2f(u);
-}
-
-// n (a multiple of 8) 16-bit values from p (16-byte aligned) into fp32
-template <bool kHalf, int N>
-__device__ __forceinline__ void load_bits(const uint16_t* p, float* x) {
-#pragma unroll
-  for (int c = 0; c < N; c += 8) {
-    const uint4 u = *reinterpret_cast<const uint4*>(p + c);
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      x[c + 2 * e] = bits_to_f32<kHalf>(uint16_t(w[e] & 0xffffu));
-      x[c + 2 * e + 1] = bits_to_f32<kHalf>(uint16_t(w[e] >> 16));
-    }
-  }
-}
-
-template <bool kHalf, int N>
-__device__ __forceinline__ void store_bits(uint16_t* p, const float* x) {
-  using FR = Frag<kHalf>;
-#pragma unroll
-  for (int c = 0; c < N; c += 8) {
-    uint4 u;
-    u.x = FR::pack(x[c], x[c + 1]);
-    u.y = FR::pack(x[c + 2], x[c + 3]);
-    u.z = FR::pack(x[c + 4], x[c + 5]);
-    u.w = FR::pack(x[c + 6], x[c + 7]);
-    *reinterpret_cast<uint4*>(p + c) = u;
-  }
-}
-
-struct BwdRows {  // one (P, A, T, HD) operand: base and element strides
-  const uint16_t* p;
-  int64_t sp, sa, st;
-  __device__ const uint16_t* row(int64_t pos, int64_t a, int64_t t) const { return p + pos * sp + a * sa + t * st; }
-};
-struct BwdOut {
-  uint16_t* p;
-  int64_t sp, sa, st;
-  __device__ uint16_t* row(int64_t pos, int64_t a, int64_t t) const { return p + pos * sp + a * sa + t * st; }
-};
-
-// Stage rows kb .. kb+63 of two operands (zeros at or past L) as fp32.
-template <bool kHalf, int HD>
-__device__ __forceinline__ void stage_pair(const BwdRows& x, const BwdRows& y, int64_t pos, int64_t a, int64_t kb,
-                                           int64_t L, float (*sx)[HD], float (*sy)[HD]) {
-  for (int i = threadIdx.x; i < kBwdChunk * HD / 8; i += 256) {
-    const int r = i / (HD / 8), c = 8 * (i % (HD / 8));
-    float vx[8], vy[8];
-    if (kb + r < L) {
-      load_bits<kHalf, 8>(x.row(pos, a, kb + r) + c, vx);
-      load_bits<kHalf, 8>(y.row(pos, a, kb + r) + c, vy);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vx[e] = vy[e] = 0.f;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      sx[r][c + e] = vx[e];
-      sy[r][c + e] = vy[e];
-    }
-  }
-}
-
-template <bool kHalf, int HD>
-__global__ void __launch_bounds__(256)
-stone_attention_bwd_q_kernel(BwdRows q, BwdRows k, BwdRows v, BwdRows o, BwdRows go, const int32_t* __restrict__ seq_lens,
-                             int heads, int64_t T, const float* __restrict__ lse, float scale,
-                             float* __restrict__ delta, BwdOut dq) {
-  using G = BwdGeom<HD>;
-  __shared__ float sk[kBwdChunk][HD], sv[kBwdChunk][HD];
-  const int64_t n_tiles = (T + G::kRows - 1) / G::kRows;
-  const int64_t pa = blockIdx.x / n_tiles, tile = blockIdx.x % n_tiles;
-  const int64_t pos = pa / heads, a = pa % heads;
-  int64_t L = seq_lens[pos];
-  L = L < 0 ? 0 : (L > T ? T : L);
-  const int64_t i = tile * G::kRows + threadIdx.x / G::kSplit;
-  const int off = (threadIdx.x % G::kSplit) * G::kDims;
-  const bool live = i < L;
-  float qv[G::kDims], gv[G::kDims], acc[G::kDims];
-  float dl = 0.f, li = 0.f;
-  if (live) {
-    float ov[G::kDims];
-    load_bits<kHalf, G::kDims>(q.row(pos, a, i) + off, qv);
-    load_bits<kHalf, G::kDims>(go.row(pos, a, i) + off, gv);
-    load_bits<kHalf, G::kDims>(o.row(pos, a, i) + off, ov);
-#pragma unroll
-    for (int d = 0; d < G::kDims; ++d) dl = fmaf(ov[d], gv[d], dl);
-    li = lse[pa * T + i];
-  } else {
-#pragma unroll
-    for (int d = 0; d < G::kDims; ++d) qv[d] = gv[d] = 0.f;
-  }
-  if constexpr (G::kSplit == 2) dl += __shfl_xor(dl, 1);
-#pragma unroll
-  for (int d = 0; d < G::kDims; ++d) acc[d] = 0.f;
-  if (tile * G::kRows < L) {  // workgroup-uniform: some row of the tile is live
-    for (int64_t kb = 0; kb < L; kb += kBwdChunk) {
-      __syncthreads();
-      stage_pair<kHalf, HD>(k, v, pos, a, kb, L, sk, sv);
-      __syncthreads();
-      const int n = int(L - kb < kBwdChunk ? L - kb : kBwdChunk);
-      for (int j = 0; j < n; ++j) {
-        float sc = 0.f, dp = 0.f;
-#pragma unroll
-        for (int d = 0; d < G::kDims; ++d) {
-          sc = fmaf(qv[d], sk[j][off + d], sc);
-          dp = fmaf(gv[d], sv[j][off + d], dp);
-        }
-        if constexpr (G::kSplit == 2) {
-          sc += __shfl_xor(sc, 1);
-          dp += __shfl_xor(dp, 1);
-        }
-        const float al = live ? expf(fmaf(sc, scale, -li)) : 0.f;
-        const float ds = al * (dp - dl);
-#pragma unroll
-        for (int d = 0; d < G::kDims; ++d) acc[d] = fmaf(ds, sk[j][off + d], acc[d]);
-      }
-    }
-  }
-  if (i < T) {
-#pragma unroll
-    for (int d = 0; d < G::kDims; ++d) acc[d] = live ? acc[d] * scale : 0.f;
-    store_bits<kHalf, G::kDims>(dq.row(pos, a, i) + off, acc);
-    if (off == 0) delta[pa * T + i] = live ? dl : 0.f;
-  }
-}
-
-template <bool kHalf, int HD>
-__global__ void __launch_bounds__(256)
-stone_attention_bwd_kv_kernel(BwdRows q, BwdRows k, BwdRows v, BwdRows go, const int32_t* __restrict__ seq_lens,
-                              int heads, int64_t T, const float* __restrict__ lse, float scale,
-                              const float* __restrict__ delta, BwdOut dk, BwdOut dv) {
-  using G = BwdGeom<HD>;
-  __shared__ float sq[kBwdChunk][HD], sg[kBwdChunk][HD];
-  __shared__ float sl[kBwdChunk], sd[kBwdChunk];
-  const int64_t n_tiles = (T + G::kRows - 1) / G::kRows;
-  const int64_t pa = blockIdx.x / n_tiles, tile = blockIdx.x % n_tiles;
-  const int64_t pos = pa / heads, a = pa % heads;
-  int64_t L = seq_lens[pos];
-  L = L < 0 ? 0 : (L > T ? T : L);
-  const int64_t j = tile * G::kRows + threadIdx.x / G::kSplit;
-  const int off = (threadIdx.x % G::kSplit) * G::kDims;
-  const bool live = j < L;
-  float kv[G::kDims], vv[G::kDims], ak[G::kDims], av[G::kDims];
-  if (live) {
-    load_bits<kHalf, G::kDims>(k.row(pos, a, j) + off, kv);
-    load_bits<kHalf, G::kDims>(v.row(pos, a, j) + off, vv);
-  } else {
-#pragma unroll
-    for (int d = 0; d < G::kDims; ++d) kv[d] = vv[d] = 0.f;
-  }
-#pragma unroll
-  for (int d = 0; d < G::kDims; ++d) ak[d] = av[d] = 0.f;
-  if (tile * G::kRows < L) {  // workgroup-uniform
-    for (int64_t qb = 0; qb < L; qb += kBwdChunk) {
-      __syncthreads();
-      stage_pair<kHalf, HD>(q, go, pos, a, qb, L, sq, sg);
-      for (int r = threadIdx.x; r < kBwdChunk; r += 256) {
-        const bool ok = qb + r < L;
-        sl[r] = ok ? lse[pa * T + qb + r] : 0.f;
-        sd[r] = ok ? delta[pa * T + qb + r] : 0.f;
-      }
-      __syncthreads();
-      const int n = int(L - qb < kBwdChunk ? L - qb : kBwdChunk);
-      for (int r = 0; r < n; ++r) {
-        float sc = 0.f, dp = 0.f;
-#pragma unroll
-        for (int d = 0; d < G::kDims; ++d) {
-          sc = fmaf(sq[r][off + d], kv[d], sc);
-          dp = fmaf(sg[r][off + d], vv[d], dp);
-        }
-        if constexpr (G::kSplit == 2) {
-          sc += __shfl_xor(sc, 1);
-          dp += __shfl_xor(dp, 1);
-        }
-        const float al = live ? expf(fmaf(sc, scale, -sl[r])) : 0.f;
-        const float ds = al * (dp - sd[r]);
-#pragma unroll
-        for (int d = 0; d < G::kDims; ++d) {
-          av[d] = fmaf(al, sg[r][off + d], av[d]);
-          ak[d] = fmaf(ds, sq[r][off + d], ak[d]);
-        }
-      }
-    }
-  }
-  if (j < T) {
-#pragma unroll
-    for (int d = 0; d < G::kDims; ++d) {
-      ak[d] = live ? ak[d] * scale : 0.f;
-      av[d] = live ? av[d] : 0.f;
-    }
-    store_bits<kHalf, G::kDims>(dk.row(pos, a, j) + off, ak);
-    store_bits<kHalf, G::kDims>(dv.row(pos, a, j) + off, av);
-  }
-}
-
 constexpr int kLatentThreads = 256;
 
 template <bool kHalf>
@@ -765,65 +545,4 @@ extern "C" int32_t mantis_stone_attention(const void* q, const int64_t* qs, cons
       ks[1], ks[2], static_cast<const uint16_t*>(v), vs[0], vs[1], vs[2], seq_lens, heads, t,
       static_cast<uint16_t*>(out), os[0], os[1], os[2], lse, c_log2, n_items, schedule);
   return launched();
-}
-
-namespace {
-template <bool kHalf, int HD>
-int32_t launch_attention_backward(const BwdRows& q, const BwdRows& k, const BwdRows& v, const BwdRows& o,
-                                  const BwdRows& go, const int32_t* seq_lens, int64_t n_pos, int heads, int64_t t,
-                                  const float* lse, float* delta, const BwdOut& dq, const BwdOut& dk,
-                                  const BwdOut& dv, hipStream_t st) {
-  using G = BwdGeom<HD>;
-  const int64_t grid = n_pos * heads * ((t + G::kRows - 1) / G::kRows);
-  if (grid > 2147483647LL) return MANTIS_E_ARG;
-  const float scale = 1.f / sqrtf(float(HD));
-  stone_attention_bwd_q_kernel<kHalf, HD><<<unsigned(grid), 256, 0, st>>>(q, k, v, o, go, seq_lens, heads, t, lse,
-                                                                          scale, delta, dq);
-  stone_attention_bwd_kv_kernel<kHalf, HD><<<unsigned(grid), 256, 0, st>>>(q, k, v, go, seq_lens, heads, t, lse,
-                                                                           scale, delta, dk, dv);
-  return launched();
-}
-}  // namespace
-
-extern "C" int32_t mantis_stone_attention_backward(const void* q, const int64_t* qs, const void* k,
-                                                   const int64_t* ks, const void* v, const int64_t* vs,
-                                                   const void* out, const int64_t* os, const void* grad_out,
-                                                   const int64_t* gs, const float* lse, int32_t dtype,
-                                                   const int32_t* seq_lens, int64_t n_pos, int32_t heads, int64_t t,
-                                                   int32_t hd, float* delta, void* dq, const int64_t* dqs, void* dk,
-                                                   const int64_t* dks, void* dv, const int64_t* dvs, void* stream) {
-  if (n_pos == 0 || t == 0) return MANTIS_OK;
-  if (!q || !k || !v || !out || !grad_out || !lse || !seq_lens || !delta || !dq || !dk || !dv) return MANTIS_E_ARG;
-  if (!qs || !ks || !vs || !os || !gs || !dqs || !dks || !dvs) return MANTIS_E_ARG;
-  if ((hd != 16 && hd != 32 && hd != 64) || heads <= 0 || n_pos < 0 || t < 0) return MANTIS_E_ARG;
-  if (dtype != MANTIS_BF16 && dtype != MANTIS_F16) return MANTIS_E_ARG;
-  // unit dim stride and 16-byte aligned rows everywhere
-  for (const int64_t* st : {qs, ks, vs, os, gs, dqs, dks, dvs}) {
-    if (st[3] != 1) return MANTIS_E_ARG;
-    if ((st[0] | st[1] | st[2]) % 8) return MANTIS_E_ARG;
-  }
-  for (const void* ptr : {q, k, v, out, grad_out, static_cast<const void*>(dq), static_cast<const void*>(dk),
-                          static_cast<const void*>(dv)})
-    if (!aligned16(ptr)) return MANTIS_E_ARG;
-  auto rows = [](const void* ptr, const int64_t* st) {
-    return BwdRows{static_cast<const uint16_t*>(ptr), st[0], st[1], st[2]};
-  };
-  auto outs = [](void* ptr, const int64_t* st) { return BwdOut{static_cast<uint16_t*>(ptr), st[0], st[1], st[2]}; };
-  const BwdRows Q = rows(q, qs), K = rows(k, ks), V = rows(v, vs), O = rows(out, os), GO = rows(grad_out, gs);
-  const BwdOut DQ = outs(dq, dqs), DK = outs(dk, dks), DV = outs(dv, dvs);
-  hipStream_t st = as_stream(stream);
-  const bool f16 = dtype == MANTIS_F16;
-#define MANTIS_BWD(H, HD_)                                                                                    \
-  return launch_attention_backward<H, HD_>(Q, K, V, O, GO, seq_lens, n_pos, heads, t, lse, delta, DQ, DK, DV, st)
-  if (hd == 16) {
-    if (f16) MANTIS_BWD(true, 16);
-    MANTIS_BWD(false, 16);
-  }
-  if (hd == 32) {
-    if (f16) MANTIS_BWD(true, 32);
-    MANTIS_BWD(false, 32);
-  }
-  if (f16) MANTIS_BWD(true, 64);
-  MANTIS_BWD(false, 64);
-#undef MANTIS_BWD
 }

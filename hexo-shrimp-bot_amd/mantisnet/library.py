@@ -64,8 +64,7 @@ def _(q, k, v, seq_lens):
 def fused_attention_backward(q: Tensor, k: Tensor, v: Tensor, seq_lens: Tensor, out: Tensor, lse: Tensor,
                              grad_out: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     """(dq, dk, dv) of fused_attention; pad rows and keys get zero gradients."""
-    dq, dk, dv = ops.stone_attention_backward(q, k, v, seq_lens, out, lse, grad_out)
-    return dq.contiguous(), dk.contiguous(), dv.contiguous()
+    return ops.stone_attention_backward(q, k, v, seq_lens, out, lse, grad_out, contiguous=True)
 
 
 @fused_attention_backward.register_fake
@@ -78,9 +77,12 @@ def _fa_setup(ctx, inputs, output) -> None:
     out, lse = output
     ctx.save_for_backward(q, k, v, seq_lens, out, lse)
     ctx.mark_non_differentiable(lse)
+    ctx.set_materialize_grads(False)  # (none is made for lse)
 
 
 def _fa_backward(ctx, grad_out, _grad_lse):
+    if grad_out is None:
+        grad_out = torch.zeros_like(ctx.saved_tensors[4])
     dq, dk, dv = fused_attention_backward(*ctx.saved_tensors, grad_out)
     return dq, dk, dv, None
 

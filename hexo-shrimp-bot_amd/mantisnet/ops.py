@@ -727,8 +727,9 @@ def latent_broadcast_backward(q, k, v, window_pos, offsets, order, m, l, grad_ou
     return _latent_backward(q, k, v, q.shape[0], k.shape[0] * 4, window_pos, offsets, order, m, l, grad_out, None)
 
 
-def stone_attention_backward(q, k, v, seq_lens, out, lse, grad_out):
-    """(dq, dk, dv) of stone_attention, in q's dtype and layout: the flash
+def stone_attention_backward(q, k, v, seq_lens, out, lse, grad_out, contiguous: bool = False):
+    """(dq, dk, dv) of stone_attention, in q's dtype and layout (or with
+    ``contiguous`` as contiguous (P, A, T, D) tensors): the flash
     backward over each position's live prefix with delta = sum(out * grad_out)
     per row (mantis_stone_attention_backward); pad rows and keys get zero
     gradients.  lse: the forward's natural-log normaliser, (P, A, T) fp32."""
@@ -751,7 +752,7 @@ def stone_attention_backward(q, k, v, seq_lens, out, lse, grad_out):
     lse, seq_lens = lse.contiguous(), seq_lens.contiguous()
 
     def like(x):
-        y = torch.empty_like(x)
+        y = torch.empty(x.shape, dtype=x.dtype, device=dev) if contiguous else torch.empty_like(x)
         return y if aligned(y) else torch.empty(x.shape, dtype=x.dtype, device=dev)
 
     dq, dk, dv = like(q), like(k), like(v)

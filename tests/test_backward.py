@@ -241,3 +241,34 @@ def test_fused_attention_backward(device, heads, hd, dt):
     again = _grads(lambda a, c, d: OPS.fused_attention(a, c, d, ld)[0], [x.to(device) for x in (q, k, v)],
                    seed.to(device, dt))
     assert all(torch.equal(a.cpu(), b.cpu()) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("hd,dt,grad_scale", [(16, torch.bfloat16, 1.0), (32, torch.bfloat16, 1.0),
+                                              (64, torch.bfloat16, 1.0), (16, torch.float16, 1.0),
+                                              (32, torch.float16, 1e-3), (64, torch.float16, 1.0)])
+def test_fused_attention_backward_tiles(device, hd, dt, grad_scale):
+    """Lengths around the 16-row sub-tiles and the 64-row tiles and chunks, T
+    off a tile, at small gradients too: within one rounding of the gradients
+    of float64 attention (2^-9 bf16, 2^-12 fp16 relative, and the forward's
+    rounded output and normaliser in delta, a few times that on the sums)."""
+    gen = torch.Generator().manual_seed(40 + hd)
+    lens = torch.tensor([0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 201], dtype=torch.int32)
+    p, t, heads = len(lens), 201, 3
+    q, k, v, go = (torch.randn(p, t, heads, hd, generator=gen).to(dt).transpose(1, 2) for _ in range(4))
+    go = (go.float() * grad_scale).to(dt)
+    valid = (torch.arange(t)[None, :] < lens[:, None])[:, None, :, None]
+    go = go.masked_fill(~valid, 0.0)
+    got = _grads(lambda a, b, c: OPS.fused_attention(a, b, c, lens.to(device))[0], [x.to(device) for x in (q, k, v)],
+                 go.to(device))
+
+    def ref(a, b, c):  # float64; a position without live rows has no keys
+        s = (a @ b.transpose(2, 3)) / hd ** 0.5
+        s = s.masked_fill(~valid.transpose(2, 3), -1e30)
+        return (s.softmax(-1) @ c).masked_fill(~valid, 0.0)
+
+    exp = _grads(ref, [x.double() for x in (q, k, v)], go.double())
+    tol = 2 ** -9 if dt == torch.bfloat16 else 2 ** -12
+    for g, e in zip(got, exp):
+        g, e = g.cpu().double(), e.masked_fill(~valid, 0.0)
+        assert float((g - e).norm() / e.norm()) < 2 * tol + 1e-7 / grad_scale
+        assert torch.count_nonzero(g.masked_fill(valid, 0.0)) == 0
