@@ -59,11 +59,13 @@ from __future__ import annotations
 
 from functools import cached_property
 
+import ctypes
+
 import torch
 import torch.nn.functional as F
 from torch import Tensor
 
-from . import ops
+from . import _hip_api, ops
 from .builder import Batch
 from .model import NEAREST_BUCKETS, RADIUS_CLASSES
 
@@ -100,6 +102,14 @@ class Prepared:
         # True while the last check found the parameters unchanged: the next
         # evaluation may then run before its check (see _speculative)
         self.steady = False
+        self._leaf = None  # (struct, its blocks, the tensors they point into)
+
+    def leaf(self):
+        """The operands as mantis_leaf_forward takes them, packed once per
+        rebuild; the pack holds every tensor it points into."""
+        if self._leaf is None:
+            self._leaf = _pack_leaf(self.model.cfg, self.t, self.params)
+        return self._leaf[0]
 
     def refresh(self):
         # the module's parameter set is fixed after construction; what changes
@@ -118,6 +128,7 @@ class Prepared:
             with torch.no_grad():
                 self.t = _prepare(self.model, {n: p.detach().float() for n, p in self.params.items()})
             self.key = key
+            self._leaf = None
         self.steady = not changed
         return changed
 
@@ -310,7 +321,52 @@ def _prepare(model, P) -> dict[str, Tensor]:
     # [hi; lo] fp16 pair of the output layer for the compensated heads
     t["head3c.w"] = ops.split_weight(w3)
     t["glin_b"] = torch.cat([P["mlp_p.lin_b.weight"], P["mlp_q.lin_b.weight"]]).contiguous()  # (256, 128)
+    t["glin_b.wt"] = t["glin_b"].t().contiguous()
+    t["mlp_v0.wt"], t["mlp_v2.wt"] = (P[f"mlp_v.{k}.weight"].t().contiguous() for k in (0, 2))
     return t
+
+
+def _pack_leaf(cfg, t, P):
+    """mantis_leaf_model over the prepared operands (and the parameters read
+    as they are), with the tensors kept alive beside it."""
+    keep = []
+
+    def ptr(x):
+        x = x.detach()
+        if x.dtype != HALF:
+            x = x.float()
+        keep.append(x.contiguous())
+        return keep[-1].data_ptr()
+
+    def block(pb):
+        vals = []
+        for name, _ in _hip_api.MantisLeafBlock._fields_:
+            if name in ("cr_bias", "radius_bias", "wr_bias"):
+                vals.append(ptr(P[pb + name]))
+            elif name in ("ws_tab", "cr_vcls", "rad_vcls"):
+                vals.append(ptr(t[pb + name]))
+            else:  # matrix "_w" / "_wt", bias "_b"
+                key, _, kind = name.rpartition("_")
+                vals.append(ptr(t[pb + key + "." + kind]))
+        return _hip_api.MantisLeafBlock(*vals)
+
+    blocks = (_hip_api.MantisLeafBlock * cfg.blocks)(*[block(f"blocks.{i}.") for i in range(cfg.blocks)])
+    m = _hip_api.MantisLeafModel(
+        blocks=ctypes.cast(blocks, ctypes.c_void_p).value, n_blocks=cfg.blocks,
+        window_table=ptr(t["window_table"]), n_patterns=t["window_table"].shape[0],
+        cell_table=ptr(t["cell_table"]), n_init=t["cell_table"].shape[0],
+        stone_table=ptr(P["stone_table.weight"]), latent_base=ptr(P["latent_base"]),
+        token_moves=ptr(P["token_moves.weight"]), sw_all=ptr(t["sw_all"]), n_occ=t["sw_all"].shape[0],
+        n_dec_classes=t["head_tab_k"].shape[0], n_rad_classes=RADIUS_CLASSES,
+        ln_out_w=ptr(P["ln_out.weight"]), ln_out_b=ptr(P["ln_out.bias"]), ln_value_w=ptr(P["ln_value.weight"]),
+        ln_value_b=ptr(P["ln_value.bias"]), value_queries=ptr(P["value_queries"]),
+        mlp_v0_wt=ptr(t["mlp_v0.wt"]), mlp_v0_b=ptr(P["mlp_v.0.bias"]), mlp_v2_wt=ptr(t["mlp_v2.wt"]),
+        mlp_v2_b=ptr(P["mlp_v.2.bias"]), n_bins=cfg.value_bins,
+        act_proj_w=ptr(t["act_proj_ln.w"]), act_proj_b=ptr(t["act_proj_ln.b"]), head1_w=ptr(t["head1ln.w"]),
+        head1_b=ptr(t["head1ln.b"]), head2_w=ptr(t["head2.w"]), head3_w=ptr(t["head3.w"]), head3_b=ptr(t["head3.b"]),
+        act_table=ptr(t["act_table16"]), n_act=t["act_table16"].shape[0], empty_rows=ptr(t["empty_rows"]),
+        head_tab=ptr(t["head_tab_k"]), glin_wt=ptr(t["glin_b.wt"]))
+    return m, blocks, keep
 
 
 def _prepared(model) -> Prepared:
@@ -923,13 +979,14 @@ def trunk(model, batch: Batch):
 
 
 def _trunk(model, b: Batch, plan: Plan, raw_cells: bool = False, W: Prepared | None = None,
-           raw_windows: bool = False):
+           raw_windows: bool = False, halves: list | None = None):
     """(w_out, g_out, cells): cells are ln_out(c) in fp16, or with raw_cells
     the fp16 cell state itself (the fused heads normalise it on the fly);
     with raw_windows, in the cell-node configuration, w_out is the fp16
     window state itself (the value read and the action projection apply
     ln_out on the fly).  W: the prepared weights when the caller has just
-    refreshed them."""
+    refreshed them.  halves: receives the heads' position half (P, 256) of
+    g_out, formed in the same launch."""
     W = W or _prepared(model)
     P = W.params
     cfg = model.cfg
@@ -984,9 +1041,11 @@ def _trunk(model, b: Batch, plan: Plan, raw_cells: bool = False, W: Prepared | N
     for i in range(cfg.blocks):
         _block(W, P, i, plan, b, sg, w, c, sw_all, i + 1 < cfg.blocks, c_init if i == 0 else None,
                w_init if i == 0 else None)
-    g = sg[n_s:].view(p, GLOBAL_ROWS, 128)
+    g = sg[n_s:]
     w_out = w if raw_windows and w.dtype == HALF else ops.layer_norm(w, P["ln_out.weight"], P["ln_out.bias"], F32)
-    g_out = F.layer_norm(g, (128,), P["ln_out.weight"], P["ln_out.bias"], 1e-5).mean(dim=1)
+    g_out, g_half = ops.latent_out(g, P["ln_out.weight"], P["ln_out.bias"], W["glin_b.wt"])
+    if halves is not None:
+        halves.append(g_half)
     if c is None:
         return w_out, g_out, None
     if not cfg.cell_nodes:
@@ -1011,7 +1070,8 @@ def value_head(model, w: Tensor, g: Tensor, batch: Batch):
 def _value_head(model, w: Tensor, g: Tensor, b: Batch, plan: Plan, W: Prepared | None = None):
     """w: ln_out(w) fp32 rows, or the raw fp16 window state (ln_out applied
     in the read)."""
-    P = (W or _prepared(model)).params
+    W = W or _prepared(model)
+    P = W.params
     if w.dtype == HALF:
         r = ops.value_read(g.float().contiguous(), w.contiguous(), plan.layout_offsets, plan.layout_order,
                            P["ln_value.weight"], P["ln_value.bias"], P["value_queries"],
@@ -1019,6 +1079,10 @@ def _value_head(model, w: Tensor, g: Tensor, b: Batch, plan: Plan, W: Prepared |
     else:
         r = ops.value_read(g.float().contiguous(), w.float().contiguous(), plan.layout_offsets, plan.layout_order,
                            P["ln_value.weight"], P["ln_value.bias"], P["value_queries"])
+    bins = model.bin_centers
+    if model.cfg.value_hidden == 128 and model.cfg.value_bins <= 128 and bins.dtype == F32:
+        return ops.value_tail(r.view(plan.n_pos, 512), W["mlp_v0.wt"], P["mlp_v.0.bias"].float(), W["mlp_v2.wt"],
+                              P["mlp_v.2.bias"].float(), bins.contiguous())
     hidden = F.relu(F.linear(r.reshape(plan.n_pos, -1), P["mlp_v.0.weight"], P["mlp_v.0.bias"]))
     logits = F.linear(hidden, P["mlp_v.2.weight"], P["mlp_v.2.bias"])
     dist = logits.softmax(-1)
@@ -1026,7 +1090,7 @@ def _value_head(model, w: Tensor, g: Tensor, b: Batch, plan: Plan, W: Prepared |
 
 
 def _head_rows(model, w: Tensor, g: Tensor, cells: Tensor, b: Batch, plan: Plan, raw_cells: bool = False,
-               W: Prepared | None = None) -> Tensor:
+               W: Prepared | None = None, g_half: Tensor | None = None) -> Tensor:
     """(N_c, 16) fp32: column 0 the policy logit, 1..3 the critic logits.
     ``cells`` are ln_out(c) rows, or with raw_cells the fp16 cell state; with
     cell state off they are None and each legal cell reads the sum of its
@@ -1048,7 +1112,8 @@ def _head_rows(model, w: Tensor, g: Tensor, cells: Tensor, b: Batch, plan: Plan,
         pre = FL(w.contiguous(), W["act_proj_ln.w"], W["act_proj_ln.b"], layer_norm=True)
     else:
         pre = FL(w.float().contiguous(), W["act_proj.w"], W["act_proj.b"])  # act_proj(w), fp16
-    g_half = F.linear(g.float(), W["glin_b"]).contiguous()  # (P, 256)
+    if g_half is None:
+        g_half = F.linear(g.float(), W["glin_b"]).contiguous()  # (P, 256)
     x = cells if cells.dtype in (HALF, F32) else cells.float()
     key = "head1ln" if raw_cells else "head1"
     tactical = None
@@ -1084,15 +1149,37 @@ def cell_heads(model, w: Tensor, g: Tensor, cells: Tensor, batch: Batch, mass_fl
 
 
 def _cell_heads(model, w, g, cells, b: Batch, plan: Plan, mass_floor: float, raw_cells: bool = False,
-                W: Prepared | None = None):
-    rows = _head_rows(model, w, g, cells, b, plan, raw_cells, W)
+                W: Prepared | None = None, g_half: Tensor | None = None):
+    rows = _head_rows(model, w, g, cells, b, plan, raw_cells, W, g_half)
     # the policy column leaves in the same pass (legal_offsets tile the cells:
     # the cell order's segment check flags them otherwise)
     policy, q_values, q_score = ops.compose_q_rows(rows, b.legal_offsets, mass_floor)
     return policy, q_score, q_values
 
 
-def _speculative(model, b: Batch, evaluate):
+# The production configuration's evaluation runs as one native call that
+# queues its launches over one workspace (True, the default), or launch by
+# launch from here (False).  The native call takes the host 0.3 ms instead of
+# 1.7-1.9, which is the whole evaluation below about 60 positions; a traced
+# evaluation (ops.trace times each launch) and every other configuration or
+# batch form run launch by launch.
+NATIVE_LEAF = True
+
+
+def _leaf_of(model, b: Batch, dev) -> _hip_api.MantisLeafBatch | None:
+    cfg = model.cfg
+    if not (NATIVE_LEAF and cfg.cell_nodes and cfg.cell_node_scope == "all" and cfg.blocks >= 1
+            and cfg.value_hidden == 128 and cfg.value_bins <= 128 and FUSE_WINDOW_PROJECTION):
+        return None
+    if cfg.cell_structure or cfg.cell_adjacency or cfg.action_tactical or SPLIT_CELL_STAGES or ops.tracing_any():
+        return None
+    bins = model.bin_centers
+    if bins.dtype != F32 or bins.device != dev or not bins.is_contiguous() or torch.cuda.current_device() != dev.index:
+        return None
+    return ops.leaf_batch(b, dev)
+
+
+def _speculative(model, b: Batch, evaluate, native):
     """Queue ``evaluate(plan, W)`` on the canonical orders the encoder emits
     and, while the parameters have been found unchanged, on the prepared
     operands of the last evaluation; both are checked once everything is
@@ -1100,18 +1187,26 @@ def _speculative(model, b: Batch, evaluate):
     check's word and the device error flag come back in one copy.  A batch in
     other orders, or parameters that changed, are evaluated again (over sorted
     tables, on rebuilt operands), the first pass's results and flags
-    discarded.  Raises ValueError on the error flag."""
+    discarded.  Raises ValueError on the error flag.  ``native(batch, W)`` is
+    the same evaluation as one native call, on the batches it takes."""
     dev = b.stone_own.device
     W, checked = _prepared_unchecked(model)
-    plan = make_plan(model, b, speculative=True)
-    out = evaluate(plan, W)
-    plan.start()  # the order check is queued (a no-op once the trunk did it)
+    leaf = _leaf_of(model, b, dev)
+    if leaf is not None:
+        out = native(leaf, W)
+    else:
+        plan = make_plan(model, b, speculative=True)
+        out = evaluate(plan, W)
+        plan.start()  # the order check is queued (a no-op once the trunk did it)
     changed = not checked and W.rebuild_if_changed()
     bits, noncanonical = ops.read_flag_and_word(dev)
     if noncanonical or changed:
         ops.error_flag(dev).zero_()
         # the same batch: a canonical one passes its check again
-        out = evaluate(make_plan(model, b, speculative=not noncanonical), W)
+        if leaf is not None and not noncanonical:
+            out = native(leaf, W)
+        else:
+            out = evaluate(make_plan(model, b, speculative=not noncanonical), W)
         bits = ops.read_flag_and_word(dev)[0]
     ops.raise_on_bits(dev, bits)
     return out
@@ -1128,12 +1223,17 @@ def forward(model, batch: Batch, mass_floor: float):
     b = batch if batch.stone_own.device == dev else batch.to(dev)
 
     def evaluate(plan, W):  # W once per evaluation: trunk and heads share it
-        w, g, c = _trunk(model, b, plan, raw_cells=True, W=W, raw_windows=True)
+        half: list = []
+        w, g, c = _trunk(model, b, plan, raw_cells=True, W=W, raw_windows=True, halves=half)
         value, value_dist, value_logits = _value_head(model, w, g, b, plan, W)
-        policy, q_score, q_values = _cell_heads(model, w, g, c, b, plan, mass_floor, raw_cells=True, W=W)
+        policy, q_score, q_values = _cell_heads(model, w, g, c, b, plan, mass_floor, raw_cells=True, W=W,
+                                                  g_half=half[0])
         return policy, q_score, q_values, value, value_dist, value_logits
 
-    return _speculative(model, b, evaluate)
+    def native(leaf, W):
+        return ops.leaf_forward(W.leaf(), leaf, model.bin_centers, mass_floor, dev)
+
+    return _speculative(model, b, evaluate, native)
 
 
 @torch.no_grad()
@@ -1146,8 +1246,12 @@ def policy_q(model, batch: Batch):
     b = batch if batch.stone_own.device == dev else batch.to(dev)
 
     def evaluate(plan, W):
-        w, g, c = _trunk(model, b, plan, raw_cells=True, W=W, raw_windows=True)
-        return _head_rows(model, w, g, c, b, plan, raw_cells=True, W=W)
+        half: list = []
+        w, g, c = _trunk(model, b, plan, raw_cells=True, W=W, raw_windows=True, halves=half)
+        return _head_rows(model, w, g, c, b, plan, raw_cells=True, W=W, g_half=half[0])
 
-    rows = _speculative(model, b, evaluate)
+    def native(leaf, W):
+        return ops.leaf_forward(W.leaf(), leaf, None, 0.0, dev)
+
+    rows = _speculative(model, b, evaluate, native)
     return rows[:, 0].contiguous(), rows[:, 1:4]

@@ -1681,6 +1681,11 @@ def tracing(name: str) -> bool:
     return _TRACE is not None and _TRACE.wants(name)
 
 
+def tracing_any() -> bool:
+    """Whether any trace is active."""
+    return _TRACE is not None
+
+
 def _strides(t: Tensor):
     return (ctypes.c_int64 * 4)(*t.stride())
 
@@ -1959,6 +1964,110 @@ def compose_q_rows(rows: Tensor, offsets: Tensor, mass_floor: float) -> tuple[Te
         _lib().mantis_compose_q_rows(_ptr(rows), rows.stride(0), _ptr(offsets), offsets.numel() - 1, n,
                                      float(mass_floor), _ptr(pol), _ptr(qv), _ptr(qs), _stream()), "compose_q"))
     return pol, qv, qs
+
+
+def latent_out(g: Tensor, gamma: Tensor, beta: Tensor, glin_wt: Tensor) -> tuple[Tensor, Tensor]:
+    """(mean of LN(g) over each position's four latents (P, 128), its product
+    with glin_wt (128, 256)), fp32; g fp32 (4 P, 128) rows."""
+    dev = _on_gpu(g, gamma, beta, glin_wt)
+    if g.dtype != torch.float32 or g.ndim != 2 or g.shape[1] != 128 or g.shape[0] % 4 or not g.is_contiguous():
+        raise ValueError("g must be contiguous fp32 (4 P, 128) rows")
+    if glin_wt.dtype != torch.float32 or glin_wt.shape != (128, 256) or not glin_wt.is_contiguous():
+        raise ValueError("glin_wt must be a contiguous fp32 (128, 256) matrix")
+    p = g.shape[0] // 4
+    g32, b32 = gamma.float().contiguous(), beta.float().contiguous()
+    out = torch.empty((p, 128), dtype=torch.float32, device=dev)
+    half = torch.empty((p, 256), dtype=torch.float32, device=dev)
+    _launch("latent_out", p * (4 * 512 + 3 * 512), p * 2 * 128 * 256, lambda: _check(
+        _lib().mantis_latent_out(_ptr(g), p, _ptr(g32), _ptr(b32), _ptr(glin_wt), _ptr(out), _ptr(half), _stream()),
+        "latent_out"))
+    return out, half
+
+
+def value_tail(read: Tensor, w0_t: Tensor, b0: Tensor, w2_t: Tensor, b2: Tensor,
+               bin_centers: Tensor) -> tuple[Tensor, Tensor, Tensor]:
+    """(value, dist, logits) of the value MLP over the reads (P, 512), fp32:
+    512 -> 128 ReLU -> n_bins <= 128, weights transposed."""
+    dev = _on_gpu(read, w0_t, b0, w2_t, b2, bin_centers)
+    p, n_bins = read.shape[0], w2_t.shape[1]
+    if any(t.dtype != torch.float32 or not t.is_contiguous() for t in (read, w0_t, b0, w2_t, b2, bin_centers)):
+        raise ValueError("value_tail takes contiguous fp32 tensors")
+    if read.shape != (p, 512) or w0_t.shape != (512, 128) or b0.shape != (128,) or w2_t.shape != (128, n_bins) \
+            or b2.shape != (n_bins,) or bin_centers.shape != (n_bins,) or not 1 <= n_bins <= 128:
+        raise ValueError("value_tail is 512 -> 128 -> up to 128 bins")
+    value = torch.empty(p, dtype=torch.float32, device=dev)
+    dist, logits = (torch.empty((p, n_bins), dtype=torch.float32, device=dev) for _ in range(2))
+    _launch("value_tail", p * 4 * (512 + 2 * n_bins) + 4 * 128 * (512 + n_bins), p * 256 * (512 + n_bins), lambda: _check(
+        _lib().mantis_value_tail(_ptr(read), p, _ptr(w0_t), _ptr(b0), _ptr(w2_t), _ptr(b2), n_bins, _ptr(bin_centers),
+                                 _ptr(value), _ptr(dist), _ptr(logits), _stream()), "value_tail"))
+    return value, dist, logits
+
+
+# ----------------------------------------------------------------- whole evaluation
+
+_LEAF_INT64 = tuple(n for n, t in _hip_api.MantisLeafBatch._fields_ if t is _hip_api.vp and n != "attn_valid")
+_LEAF_LENGTHS = {  # entries of each table, by the size it has to match
+    "n_s": ("stone_slot",), "n_w": ("window_slot",), "n_pos": ("moves_idx",), "n_c": ("cell_nearest",),
+    "n_inc": ("inc_window", "inc_class"), "n_rad": ("radius_dst", "radius_orbit", "radius_own", "radius_on_axis"),
+    "n_dec": ("dec_window", "dec_class", "act_class", "act_rev")}
+
+
+def leaf_batch(b, dev: torch.device) -> _hip_api.MantisLeafBatch | None:
+    """The batch as mantis_leaf_forward takes it: contiguous int64 tables of
+    matching lengths on the device, every size at least 1, the covered cells
+    counted by the relay views.  None for any other batch (the launch-by-launch
+    composition takes or refuses those)."""
+    idx = dev.index if dev.index is not None else torch.cuda.current_device()
+    ptrs = []
+    for name in _LEAF_INT64:
+        t = getattr(b, name)
+        if t.dtype is not torch.int64 or t.get_device() != idx or not t.is_contiguous() or not t.numel():
+            return None
+        ptrs.append(t.data_ptr())
+    valid, relay = b.attn_valid, getattr(b, "relay_cell_ptr", None)
+    if relay is None or valid.dtype is not torch.bool or valid.get_device() != idx or not valid.is_contiguous():
+        return None
+    if valid.ndim != 2 or b.value_valid.ndim != 2:
+        return None
+    (n_pos, max_t), max_w = valid.shape, b.value_valid.shape[1]
+    sizes = {"n_s": b.stone_own.numel(), "n_w": b.window_feat.numel(), "n_pos": n_pos, "n_c": b.cell_pos.numel(),
+             "n_inc": b.inc_stone.numel(), "n_rad": b.radius_src.numel(), "n_dec": b.dec_cell.numel()}
+    if any(getattr(b, t).numel() != sizes[k] for k, ts in _LEAF_LENGTHS.items() for t in ts):
+        return None
+    n_cov = relay.numel() - 1
+    if b.legal_offsets.numel() != n_pos + 1 or b.act_empty.numel() != 3 * sizes["n_c"] or n_cov < 1 \
+            or not 4 <= max_t <= 2048 or n_pos * max_t >= 2**31 or max_w < 1 or max(sizes.values()) >= 2**31:
+        return None
+    return _hip_api.MantisLeafBatch(*ptrs, valid.data_ptr(), n_pos, max_t, max_w, sizes["n_s"], sizes["n_w"],
+                                    sizes["n_c"], n_cov, sizes["n_inc"], sizes["n_rad"], sizes["n_dec"])
+
+
+def leaf_forward(model: _hip_api.MantisLeafModel, batch: _hip_api.MantisLeafBatch, bin_centers: Tensor | None,
+                 mass_floor: float, dev: torch.device):
+    """One evaluation as one native call (mantis_leaf_forward): with
+    bin_centers (policy, q_score, q_values, value, value_dist, value_logits),
+    else the head rows (n_c, 4).  The order check's word and the error flag
+    are left in the device's two words."""
+    lib, bb = _lib(), ctypes.byref(batch)
+    need = lib.mantis_leaf_workspace(bb, model.n_blocks)
+    if need < 0:
+        raise ValueError("leaf_forward: unsupported batch sizes")
+    n_c, p, n_bins = batch.n_c, batch.n_pos, model.n_bins
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    rows = torch.empty((n_c, 4), dtype=torch.float32, device=dev)
+    out = _hip_api.MantisLeafOut(rows=rows.data_ptr())
+    res = rows
+    if bin_centers is not None:
+        policy, q_values, q_score = (torch.empty(n_c, dtype=torch.float32, device=dev) for _ in range(3))
+        value = torch.empty(p, dtype=torch.float32, device=dev)
+        dist, logits = (torch.empty((p, n_bins), dtype=torch.float32, device=dev) for _ in range(2))
+        out = _hip_api.MantisLeafOut(bin_centers.data_ptr(), rows.data_ptr(), policy.data_ptr(), q_values.data_ptr(),
+                                     q_score.data_ptr(), value.data_ptr(), dist.data_ptr(), logits.data_ptr())
+        res = policy, q_score, q_values, value, dist, logits
+    flag = _flag_words(dev).data_ptr()
+    _check(lib.mantis_leaf_forward(ctypes.byref(model), bb, ctypes.byref(out), float(mass_floor), ws.data_ptr(), need,
+                                   flag + 4, flag, _ptr(tile_counters(dev)), _stream()), "leaf_forward")
+    return res
 
 
 # ----------------------------------------------------------------- hex message passing

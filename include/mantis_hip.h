@@ -988,6 +988,200 @@ int32_t mantis_hex_aggregate_linear(const void* x, const int32_t* nbr, int64_t n
                                     const void* w, const float* b, void* out_sum, void* out_mean,
                                     int32_t* err_flag, void* stream);
 
+/*
+ * The latent rows' output: g (4 n_pos, 128) fp32 through LayerNorm (gamma,
+ * beta), each position's mean into g_out (n_pos, 128) and its product with
+ * glin_wt (128, 256) into g_half (n_pos, 256).  Replaces ln_out(g).mean and
+ * the heads' lin_b of it (model.py:975-985, 1111-1139).
+ */
+int32_t mantis_latent_out(const float* g, int64_t n_pos, const float* gamma, const float* beta, const float* glin_wt,
+                          float* g_out, float* g_half, void* stream);
+
+/*
+ * The value MLP of the four-query reads (n_pos, 512): hidden = relu(w0 x + b0)
+ * (128 wide, w0_t (512, 128)), logits = w2 hidden + b2 (w2_t (128, n_bins),
+ * n_bins <= 128), dist their softmax and value its mean over bin_centers, all
+ * fp32.  Replaces mlp_v and the readout of value_head (model.py:1175-1183).
+ */
+int32_t mantis_value_tail(const float* read, int64_t n_pos, const float* w0_t, const float* b0, const float* w2_t,
+                          const float* b2, int64_t n_bins, const float* bin_centers, float* value, float* dist,
+                          float* logits, void* stream);
+
+/*
+ * One leaf evaluation of the production network (cell nodes over every legal
+ * cell, H = 128, 4 heads) as one call: the index plan, the trunk, the value
+ * head and the cell heads, each launch of the composition above queued on
+ * `stream` without a host round trip (MantisNet.forward, model.py:898-1200).
+ * The batch must be in the encoder's canonical orders; *noncanonical (device)
+ * is set nonzero if it is not, and the results are then meaningless.  Index
+ * errors are flagged in err_flag as by the launches themselves.
+ *
+ * mantis_leaf_batch: the batch's device tables (contiguous int64, attn_valid
+ * bytes) and sizes, all at least 1; n_cov the cells with decoder entries.
+ * mantis_leaf_block / mantis_leaf_model: the prepared weights: matrices fp16
+ * with the preceding LayerNorm folded in where one precedes, biases and
+ * tables fp32 unless noted.
+ * mantis_leaf_out: rows (n_c, 4) fp32 head rows, always written; with value
+ * non-NULL also policy, q_values, q_score (n_c) and value (n_pos), dist and
+ * logits (n_pos, n_bins).
+ * workspace: mantis_leaf_workspace(batch, n_blocks) bytes, 256-byte
+ * aligned.
+ */
+typedef struct mantis_leaf_batch {
+  const int64_t* stone_own;
+  const int64_t* window_feat;
+  const int64_t* moves_idx;
+  const int64_t* inc_stone;
+  const int64_t* inc_window;
+  const int64_t* inc_class;
+  const int64_t* stone_slot;
+  const int64_t* window_slot;
+  const int64_t* legal_offsets;
+  const int64_t* cell_pos;
+  const int64_t* cell_nearest;
+  const int64_t* radius_src;
+  const int64_t* radius_dst;
+  const int64_t* radius_orbit;
+  const int64_t* radius_own;
+  const int64_t* radius_on_axis;
+  const int64_t* dec_cell;
+  const int64_t* dec_window;
+  const int64_t* dec_class;
+  const int64_t* act_class;
+  const int64_t* act_rev;
+  const int64_t* act_empty;
+  const uint8_t* attn_valid;
+  int64_t n_pos;
+  int64_t max_t;
+  int64_t max_w;
+  int64_t n_s;
+  int64_t n_w;
+  int64_t n_c;
+  int64_t n_cov;
+  int64_t n_inc;
+  int64_t n_rad;
+  int64_t n_dec;
+} mantis_leaf_batch;
+
+typedef struct mantis_leaf_block {
+  const void* u_w;
+  const float* u_b;
+  const void* mlp_w1_w;
+  const float* mlp_w1_b;
+  const void* mlp_w2_w;
+  const float* ws_tab;
+  const void* mlp_w3_w;
+  const float* mlp_w3_b;
+  const void* cr_kv_w;
+  const float* cr_kv_b;
+  const void* cr_q_w;
+  const float* cr_q_b;
+  const void* cr_o_w;
+  const float* cr_o_b;
+  const float* cr_bias;
+  const void* cr_vcls;
+  const void* rad_kv_w;
+  const float* rad_kv_b;
+  const void* rad_q_w;
+  const float* rad_q_b;
+  const void* rad_o_w;
+  const float* rad_o_b;
+  const float* radius_bias;
+  const void* rad_vcls;
+  const void* wr_kv_w;
+  const float* wr_kv_b;
+  const void* wr_q_w;
+  const float* wr_q_b;
+  const void* wr_o_w;
+  const float* wr_o_b;
+  const float* wr_bias;
+  const void* wproj_w;
+  const float* wproj_b;
+  const void* mlp_s1_w;
+  const float* mlp_s1_b;
+  const void* mlp_s2_w;
+  const void* mlp_s3_w;
+  const float* mlp_s3_b;
+  const void* qkv_w;
+  const float* qkv_b;
+  const void* attn_o_w;
+  const float* attn_o_b;
+  const void* lq_read_x_w;
+  const float* lq_read_x_b;
+  const void* lread_v_w;
+  const float* lread_v_b;
+  const void* lo_read_w;
+  const float* lo_read_b;
+  const float* mix_qkv_wt;
+  const float* mix_qkv_b;
+  const float* mix_o_wt;
+  const float* mix_o_b;
+  const void* lkv_bcast_w;
+  const float* lkv_bcast_b;
+  const void* bcast_q_w;
+  const float* bcast_q_b;
+  const void* lo_bcast_w;
+  const float* lo_bcast_b;
+  const void* ffn1_w;
+  const float* ffn1_b;
+  const void* ffn2_w;
+  const float* ffn2_b;
+} mantis_leaf_block;
+
+typedef struct mantis_leaf_model {
+  const mantis_leaf_block* blocks;
+  int64_t n_blocks;
+  const void* window_table; /* fp16 (n_patterns, 128) */
+  int64_t n_patterns;
+  const void* cell_table; /* fp16 (n_init, 128), the covered cells' row last */
+  int64_t n_init;
+  const float* stone_table; /* (2, 128) */
+  const float* latent_base; /* (4, 128) */
+  const float* token_moves; /* (2, 128) */
+  const float* sw_all;      /* (n_occ, 128 n_blocks) */
+  int64_t n_occ;
+  int64_t n_dec_classes;
+  int64_t n_rad_classes;
+  const float* ln_out_w;
+  const float* ln_out_b;
+  const float* ln_value_w;
+  const float* ln_value_b;
+  const float* value_queries; /* (4, 128) */
+  const float* mlp_v0_wt;     /* (512, 128) */
+  const float* mlp_v0_b;
+  const float* mlp_v2_wt; /* (128, n_bins) */
+  const float* mlp_v2_b;
+  int64_t n_bins;
+  const void* act_proj_w;
+  const float* act_proj_b;
+  const void* head1_w;
+  const float* head1_b;
+  const void* head2_w;
+  const void* head3_w;
+  const float* head3_b;
+  const void* act_table; /* fp16 (n_act, 128) */
+  int64_t n_act;
+  const float* empty_rows; /* (3, 128) */
+  const void* head_tab;    /* fp16, quad-chunked (n_dec_classes, 256) */
+  const float* glin_wt;    /* (128, 256) */
+} mantis_leaf_model;
+
+typedef struct mantis_leaf_out {
+  const float* bin_centers;
+  float* rows;
+  float* policy;
+  float* q_values;
+  float* q_score;
+  float* value;
+  float* dist;
+  float* logits;
+} mantis_leaf_out;
+
+int64_t mantis_leaf_workspace(const mantis_leaf_batch* batch, int64_t n_blocks);
+int32_t mantis_leaf_forward(const mantis_leaf_model* model, const mantis_leaf_batch* batch,
+                            const mantis_leaf_out* out, float mass_floor, void* workspace, int64_t workspace_bytes,
+                            int32_t* noncanonical, int32_t* err_flag, uint32_t* tile_counters, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

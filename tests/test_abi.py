@@ -52,6 +52,16 @@ def test_substage_struct_matches_header():
     assert ctypes.sizeof(_hip_api.MantisSubstage) == 8 * len(fields)
 
 
+@pytest.mark.parametrize("name", ["batch", "block", "model", "out"])
+def test_leaf_structs_match_header(name):
+    text = (INCLUDE / "mantis_hip.h").read_text()
+    body = re.search(rf"typedef struct mantis_leaf_{name} \{{(.*?)\}} mantis_leaf_{name};", text, flags=re.S).group(1)
+    body = re.sub(r"/\*.*?\*/", "", body, flags=re.S)
+    struct = getattr(_hip_api, f"MantisLeaf{name.capitalize()}")
+    assert re.findall(r"(\w+);", body) == [f for f, _ in struct._fields_]
+    assert ctypes.sizeof(struct) == 8 * len(struct._fields_)
+
+
 def test_versions_answer_without_a_gpu():
     assert _native.encoder().hexo_repr_version() == 9
     assert _native.hip().mantis_hip_version() > 0

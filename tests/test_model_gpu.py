@@ -306,6 +306,75 @@ def test_weights_changed_between_evaluations_are_used(device):
         assert _same_outputs(got, fresh(batch, 0.2))
 
 
+@pytest.mark.parametrize("config,count", [(1, 1), (4, 1), (4, 9), (5, 2)])
+def test_native_leaf_is_bitwise_the_launch_by_launch_evaluation(device, config, count):
+    # one native call over one workspace against the same launches queued from
+    # Python: every output of the forward, and the evaluator's head rows
+    from mantisnet import forward, ops
+
+    net = _model(device, PRODUCTION, seed=6)
+    batch = collate_positions(synthetic.random_games(config, count, start=700)).to(device)
+    outs = []
+    saved = forward.NATIVE_LEAF
+    try:
+        for native in (True, False):
+            forward.NATIVE_LEAF = native
+            assert (forward._leaf_of(net, batch, batch.stone_own.device) is not None) == native
+            with torch.no_grad():
+                out = net(batch, 0.2)
+                outs.append([getattr(out, n) for n in ("policy_logits", "q_score", "q_values", "value", "value_dist",
+                                                       "value_logits")] + list(forward.policy_q(net, batch)))
+            ops.raise_on_device_error(device)
+    finally:
+        forward.NATIVE_LEAF = saved
+    for a, b in zip(*outs):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
+def test_native_leaf_takes_only_the_batches_it_is_built_for(device):
+    # empty tables, other dtypes and lengths that disagree go to the
+    # launch-by-launch composition; a bad stone owner raises
+    import dataclasses
+
+    from mantisnet import forward, ops
+
+    net = _model(device, PRODUCTION, seed=6)
+    batch = collate_positions(synthetic.random_games(4, 3, start=710)).to(device)
+    dev = batch.stone_own.device
+    assert forward._leaf_of(net, batch, dev) is not None
+    for change in (dict(stone_own=batch.stone_own.int()), dict(act_class=batch.act_class[:-1]),
+                   dict(radius_src=batch.radius_src[:0]), dict(relay_cell_ptr=None),
+                   dict(window_feat=batch.window_feat.repeat_interleave(2)[::2])):
+        assert forward._leaf_of(net, dataclasses.replace(batch, **change), dev) is None
+    own = batch.stone_own.clone()
+    own[1] = 2
+    with pytest.raises(ValueError), torch.no_grad():
+        net(dataclasses.replace(batch, stone_own=own), 0.2)
+    ops.raise_on_device_error(device)  # nothing is left for the next call
+
+
+def test_value_tail_and_latent_out_match_torch(device):
+    # around the four positions of a workgroup and the wavefront's 64 bins
+    from mantisnet import ops
+
+    gen = torch.Generator().manual_seed(31)
+    for p, n_bins in ((1, 1), (3, 64), (4, 65), (5, 128)):
+        r = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+        read, w0, b0, w2, b2, bins = r(p, 512), r(128, 512) / 22, r(128), r(n_bins, 128) / 11, r(n_bins), r(n_bins)
+        g, gamma, beta, glin = r(4 * p, 128), r(128), r(128), r(256, 128) / 11
+        d = lambda t: t.to(device)  # noqa: E731
+        value, dist, logits = ops.value_tail(d(read), d(w0.t().contiguous()), d(b0), d(w2.t().contiguous()), d(b2), d(bins))
+        x = (torch.relu(read.double() @ w0.double().t() + b0.double()) @ w2.double().t() + b2.double())
+        # fp32 sums of 512 and 128 products near 1
+        torch.testing.assert_close(logits.cpu().double(), x, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(dist.cpu().double(), x.softmax(-1), rtol=1e-4, atol=1e-6)
+        torch.testing.assert_close(value.cpu().double(), x.softmax(-1) @ bins.double(), rtol=1e-4, atol=1e-5)
+        out, half = ops.latent_out(d(g), d(gamma), d(beta), d(glin.t().contiguous()))
+        exp = torch.nn.functional.layer_norm(g.double(), (128,), gamma.double(), beta.double(), 1e-5).view(p, 4, 128).mean(1)
+        torch.testing.assert_close(out.cpu().double(), exp, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(half.cpu().double(), exp @ glin.double().t(), rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("knobs", [dict(), dict(cell_latents=True, cell_nodes=False)])
 def test_fused_window_projection_is_bitwise_the_separate_launch(device, knobs):
     # the windows <- cells sub-stage forming the stones <- windows value
