@@ -859,7 +859,10 @@ int32_t mantis_run_reduce(const void* values, int32_t values_dtype, int64_t n_sr
     using TI = decltype(ti);
     out_ok = with_type(out_dtype, [&](auto to) {
       using TO = decltype(to);
-      if (vec && h == 128 && n_src > 0)
+      // 128-wide rows of short runs (a window's 1.1 stones): two rows per group,
+      // an entry at a time.  From 4 entries a run on (a stone's 18 windows), 16
+      // indices per load and 4 rows in flight; the sums are the same in both.
+      if (vec && h == 128 && n_src > 0 && n_entries < 4 * n_dest)
         run_reduce_rows_kernel<TI, TO><<<dim3(unsigned((n_dest + kGroupsPerBlock * kRowsRR - 1) /
                                                         (kGroupsPerBlock * kRowsRR))),
                                          block, 0, s>>>(static_cast<const TI*>(values), n_src, ld, gather, ptr,
