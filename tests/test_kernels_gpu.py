@@ -484,6 +484,29 @@ def _hex_graphs(n_graphs, seed=0):
     return games, cells, sizes
 
 
+@pytest.mark.parametrize("sizes", [[1], [0, 3, 0, 0, 1, 255], [256, 256, 1], [300] * 7, [1] * 700, [5000, 40, 3100],
+                                   [2] * 5000 + [600]])
+def test_hex_neighbours_graph_sizes(device, sizes):
+    """Empty and single-cell graphs, graphs around a 256-cell workgroup and
+    past the 3,072 staged cells, more graphs than one round of 64 x 64 probes:
+    the table by a dictionary."""
+    gen = torch.Generator().manual_seed(50 + len(sizes))
+    cells, nbr, base = [], [], 0
+    for n in sizes:
+        side = max(2, int(n ** 0.5 * 1.3) + 1)
+        pick = torch.randperm(side * side, generator=gen)[:n].sort().values
+        own = [(int(k) // side - 3, int(k) % side - 5) for k in pick]
+        at = {c: base + j for j, c in enumerate(own)}
+        for q, r in own:
+            nbr.append([at.get((q + dq, r + dr), -1) for dq, dr in ((1, 0), (-1, 0), (0, 1), (0, -1), (1, -1), (-1, 1))])
+        cells += own
+        base += n
+    ptr = torch.tensor([0] + sizes).cumsum(0)
+    got = ops.hex_neighbours(torch.tensor(cells, dtype=torch.int32).to(device), ptr.to(device))
+    ops.raise_on_device_error(device)
+    assert torch.equal(got.cpu(), torch.tensor(nbr, dtype=torch.int32))
+
+
 def test_hex_neighbours_bit_exact_vs_reference_adjacency(device):
     games, cells, sizes = _hex_graphs(6)
     qr = torch.from_numpy(np.concatenate(cells).astype(np.int32))
