@@ -66,7 +66,7 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from . import _hip_api, ops
-from .builder import Batch
+from .builder import RELAY_FIELDS, Batch
 from .model import NEAREST_BUCKETS, RADIUS_CLASSES
 
 HALF = torch.float16
@@ -735,13 +735,35 @@ def make_plan(model, b: Batch, speculative: bool = False) -> Plan:
     return Plan(model, b, speculative)
 
 
+def batch_on(model, batch: Batch, device) -> Batch:
+    """The batch with the tables that ``model`` reads on ``device``; the others
+    stay where they are: the window and stone coordinates, the adjacency edges,
+    the relay views (their length counts the covered cells), the tactical
+    scalars and the value mask (its width alone is read) belong to other
+    configurations or to none.  A host batch's copies (the search's, the PyO3
+    seam's) bound a small evaluation: 24 positions of 40-120 stones are 47 MB,
+    27 of them read in the production configuration (3,470 -> 2,630 us through
+    the evaluator seam)."""
+    cfg = model.cfg
+    unread = {"window_id", "coords", "value_valid", "adjacency_axis"}
+    if not (cfg.cell_nodes and cfg.cell_adjacency):
+        unread |= {"adjacency_src", "adjacency_dst"}
+    if not cfg.action_tactical:
+        unread.add("act_tactical")
+    if cfg.uses_cell_state:
+        unread |= set(RELAY_FIELDS)
+    moved = {k: (v.to(device, non_blocking=True) if isinstance(v, Tensor) and k not in unread else v)
+             for k, v in vars(batch).items()}
+    return Batch(**moved)
+
+
 def _plan_for(model, batch: Batch) -> tuple[Batch, Plan]:
     """The batch on the model's device and its index plan, derived afresh on
     every call (nothing is kept on the model, so a batch refilled in place
     never meets a stale plan).  A batch on another device (the PyO3 seam builds
     CPU tensors) is moved first."""
     dev = next(model.parameters()).device
-    b = batch if batch.stone_own.device == dev else batch.to(dev)
+    b = batch if batch.stone_own.device == dev else batch_on(model, batch, dev)
     return b, make_plan(model, b)
 
 
@@ -1220,7 +1242,7 @@ def forward(model, batch: Batch, mass_floor: float):
     weights.  Index errors the kernels flagged raise ValueError."""
     _supported(model)
     dev = next(model.parameters()).device
-    b = batch if batch.stone_own.device == dev else batch.to(dev)
+    b = batch if batch.stone_own.device == dev else batch_on(model, batch, dev)
 
     def evaluate(plan, W):  # W once per evaluation: trunk and heads share it
         half: list = []
@@ -1243,7 +1265,7 @@ def policy_q(model, batch: Batch):
     value readout.  Same plan, fused heads over the raw cell state and device
     error check as ``forward``: (policy logits (N_c,), critic logits (N_c, 3))."""
     dev = _supported(model)
-    b = batch if batch.stone_own.device == dev else batch.to(dev)
+    b = batch if batch.stone_own.device == dev else batch_on(model, batch, dev)
 
     def evaluate(plan, W):
         half: list = []

@@ -49,11 +49,13 @@ _gpu_lock = threading.Lock()
 
 
 def network_evaluate(model, cfg: KlentConfig):
-    """The evaluator closure (train.py:100-120)."""
+    """The evaluator closure (train.py:100-120).  Of a host batch only the
+    tables that the model reads go to the device."""
+    from .. import forward as fwd
 
     def evaluate(batch):
         with _gpu_lock:
-            b = batch.to(cfg.device)
+            b = fwd.batch_on(model, batch, cfg.device)
             with torch.no_grad():
                 policy, critic_logits = _policy_q(model, b)
                 # both Q roles from one launch: (compose_q, compose_acting_q)

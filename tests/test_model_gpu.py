@@ -169,6 +169,23 @@ def test_network_evaluate_seam(device):
     assert (q_values - ref["q_values"]).abs().max() <= 1e-2
 
 
+@pytest.mark.parametrize("knobs", [dict(), dict(cell_latents=True, cell_nodes=True, cell_adjacency=True,
+                                                action_tactical=True),
+                                   dict(cell_latents=True, cell_nodes=False), dict(cell_nodes=False)])
+def test_a_host_batch_takes_only_the_tables_its_model_reads(device, knobs):
+    # every configuration evaluates a host batch as the same batch moved whole
+    from mantisnet import forward
+
+    net = _model(device, MantisConfig(**knobs) if knobs else PRODUCTION, seed=7)
+    batch = collate_positions(synthetic.random_games(4, 4, start=720))
+    moved = forward.batch_on(net, batch, device)
+    assert moved.stone_own.is_cuda and not moved.coords.is_cuda and moved.act_tactical.is_cuda == net.cfg.action_tactical
+    with torch.no_grad():
+        a, b, c = net(batch, 0.2), net(batch.to(device), 0.2), net(moved, 0.2)
+    for name in ("policy_logits", "q_score", "q_values", "value"):
+        assert torch.equal(getattr(a, name), getattr(b, name)) and torch.equal(getattr(a, name), getattr(c, name))
+
+
 def test_network_evaluate_equals_the_forward_heads(device):
     # the seam's fused evaluation gives bitwise the forward's policy and Q
     net = _model(device, seed=2)
