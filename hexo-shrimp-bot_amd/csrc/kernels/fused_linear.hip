@@ -126,6 +126,12 @@ template <typename TX, typename TX2, bool kLN, int N1, bool kX2, bool kRelu, boo
           bool kSplit = false, bool kPair = false>
 __global__ void __launch_bounds__((threads_for<N1, kX2, kStage2>())) fused_linear_kernel(Args a) {
   static_assert(!kPair || (!kStage2 && !kX2 && kMode == kStoreF16 && N1 % 32 == 0), "paired stores: fp16 projections");
+  // a projection of few rows: grid row y takes output columns N1 y .. (launch_columns)
+  if constexpr (kPair) {
+    a.w1 += blockIdx.y * (N1 * kK);
+    if (a.b1) a.b1 += blockIdx.y * N1;
+    a.out = static_cast<_Float16*>(a.out) + blockIdx.y * N1;
+  }
   constexpr int kTileRows = 16 * (threads_for<N1, kX2, kStage2>() / 64);
   constexpr int kParts = kSplit ? 2 : 1;
   // The fp16 in-place residual MLP (the window pair MLP): stage 2's outputs
@@ -538,7 +544,7 @@ int cu_count() {
 
 template <typename TX, typename TX2, bool kLN, int N1, bool kX2, bool kRelu, bool kStage2, int kMode,
           bool kSplit = false, bool kPair = false>
-int32_t launch(const Args& a, hipStream_t stream) {
+int32_t launch(const Args& a, hipStream_t stream, int columns = 1) {
   using S = Smem<N1, kStage2, kX2, kSplit>;
   auto kernel = fused_linear_kernel<TX, TX2, kLN, N1, kX2, kRelu, kStage2, kMode, kSplit, kPair>;
   const int bytes = S::bytes(a.n3);
@@ -554,8 +560,25 @@ int32_t launch(const Args& a, hipStream_t stream) {
   const int64_t tiles = (a.m + kTileRows - 1) / kTileRows;
   const int per_cu = std::max(1, std::min(4, kMaxLds / std::max(bytes, 1)));
   const int64_t grid = std::min<int64_t>(tiles, int64_t(cu_count()) * per_cu);
-  kernel<<<unsigned(grid), threads_for<N1, kX2, kStage2>(), bytes, stream>>>(a);
+  kernel<<<dim3(unsigned(grid), unsigned(columns)), threads_for<N1, kX2, kStage2>(), bytes, stream>>>(a);
   return launched();
+}
+
+// A LayerNorm'd projection to fp16 rows, n1 wide (a multiple of 128).  A
+// workgroup stages all the weights of its columns before its first row (64 KB
+// for 256 columns, 128 KB for 512), which is most of a launch over a few
+// hundred rows, so a launch that leaves CUs idle cuts its columns over grid
+// rows of 64 or 128 as long as every workgroup then has a CU of its own.  Each
+// output is computed as before.  (512 wide over the four latent rows of one
+// position: 13.3 us uncut, 4.6 cut; 2,048 rows 17.8 and 6.2.)
+template <typename TX, int N1>
+int32_t launch_columns(const Args& a, hipStream_t s) {
+  const int64_t tiles = (a.m + 127) / 128;  // rows of a 512-thread workgroup
+  const int64_t cus = cu_count();
+  if (tiles * (N1 / 64) <= cus) return launch<TX, float, true, 64, false, false, false, 0, false, true>(a, s, N1 / 64);
+  if (N1 > 128 && tiles * (N1 / 128) <= cus)
+    return launch<TX, float, true, 128, false, false, false, 0, false, true>(a, s, N1 / 128);
+  return launch<TX, float, true, N1, false, false, false, 0, false, true>(a, s);
 }
 
 }  // namespace
@@ -620,10 +643,10 @@ extern "C" int32_t mantis_fused_linear(const void* x, int32_t x_dtype, int64_t l
     // the projections (fp16 out; paired 16-byte stores, except where an
     // add1/add2 row is read per feature)
     if (x_dtype == MANTIS_F32 && ln && !r && mode == 0 && !a.add1 && !a.add2) {
-      if (n1 == 128) return launch<float, float, true, 128, false, false, false, 0, false, true>(a, s);
-      if (n1 == 256) return launch<float, float, true, 256, false, false, false, 0, false, true>(a, s);
-      if (n1 == 384) return launch<float, float, true, 384, false, false, false, 0, false, true>(a, s);
-      if (n1 == 512) return launch<float, float, true, 512, false, false, false, 0, false, true>(a, s);
+      if (n1 == 128) return launch_columns<float, 128>(a, s);
+      if (n1 == 256) return launch_columns<float, 256>(a, s);
+      if (n1 == 384) return launch_columns<float, 384>(a, s);
+      if (n1 == 512) return launch_columns<float, 512>(a, s);
     }
     if (x_dtype == MANTIS_F32 && ln && !r && mode == 0) {
       if (n1 == 128) return launch<float, float, true, 128, false, false, false, 0>(a, s);
@@ -636,13 +659,13 @@ extern "C" int32_t mantis_fused_linear(const void* x, int32_t x_dtype, int64_t l
     // fp16 rows with a LayerNorm (the cell state's k/v projection; the
     // heads' action projection of the raw window state)
     if (x_dtype == MANTIS_F16 && ln && !r && mode == 0 && n1 == 128 && !a.add1 && !a.add2)
-      return launch<_Float16, float, true, 128, false, false, false, 0, false, true>(a, s);
+      return launch_columns<_Float16, 128>(a, s);
     if (x_dtype == MANTIS_F16 && ln && !r && mode == 0 && n1 == 256 && !a.add1 && !a.add2)
-      return launch<_Float16, float, true, 256, false, false, false, 0, false, true>(a, s);
+      return launch_columns<_Float16, 256>(a, s);
     if (x_dtype == MANTIS_F16 && ln && !r && mode == 0 && n1 == 384 && !a.add1 && !a.add2)
-      return launch<_Float16, float, true, 384, false, false, false, 0, false, true>(a, s);
+      return launch_columns<_Float16, 384>(a, s);
     if (x_dtype == MANTIS_F16 && ln && !r && mode == 0 && n1 == 512 && !a.add1 && !a.add2)
-      return launch<_Float16, float, true, 512, false, false, false, 0, false, true>(a, s);
+      return launch_columns<_Float16, 512>(a, s);
     if (x_dtype == MANTIS_F16 && ln && !r && mode == 0 && n1 == 256)
       return launch<_Float16, float, true, 256, false, false, false, 0>(a, s);
     if (!ln && !r && mode == 2 && n1 == 128) {

@@ -936,6 +936,33 @@ def test_latent_read_from_the_window_rows_matches_the_projected_read(device):
     ops.raise_on_device_error(device)
 
 
+@pytest.mark.parametrize("n1", [128, 256, 384, 512])
+@pytest.mark.parametrize("dt", [torch.float32, H16])
+def test_few_row_projections_cut_by_columns_are_bitwise_the_whole(device, n1, dt):
+    # columns cut over grid rows of 64 (a few rows) or 128 (thousands), against
+    # the same rows inside a launch too long to cut
+    gen = _g(17)
+    x = torch.randn(40000, 128, generator=gen).to(dt).to(device)
+    w = (torch.randn(n1, 128, generator=gen) / 11).to(H16).to(device)
+    b = torch.randn(n1, generator=gen).to(device)
+    whole = ops.fused_linear(x, w, b, layer_norm=True)
+    for m in (1, 4, 129, 4100, 8300, 16384, 16385):
+        assert torch.equal(ops.fused_linear(x[:m], w, b, layer_norm=True), whole[:m])
+        rows = torch.arange(m, device=device).flip(0)
+        assert torch.equal(ops.fused_linear(x, w, b, layer_norm=True, x_rows=rows), whole[:m].flip(0))
+
+
+def test_latent_mix_over_more_positions_than_workgroups(device):
+    # 1,100 positions (1,024 workgroups at most): each as in a launch of its own
+    gen = _g(18)
+    g = torch.randn(4400, 128, generator=gen).to(device)
+    w, wo = (torch.randn(128, n, generator=gen).to(device) / 11 for n in (384, 128))
+    b, bo = (torch.randn(n, generator=gen).to(device) for n in (384, 128))
+    whole = ops.latent_mix(g.clone(), w, b, wo, bo)
+    assert torch.equal(ops.latent_mix(g[:4].clone(), w, b, wo, bo), whole[:4])
+    assert torch.equal(ops.latent_mix(g[4096:].clone(), w, b, wo, bo), whole[4096:])
+
+
 def test_latent_mix_matches_the_fp32_formulation(device):
     # the four latents of a position attend to each other (model.py:516-526)
     gen = _g(13)
