@@ -2,23 +2,29 @@
 // the class gradients' counterpart of argsort(key, stable) + gather + CSR, in
 // three launches for up to 2,048 keys.
 //
-//   count    each wavefront counts the keys of its tile of 1,024 entries in LDS
-//   scan     per key, the exclusive prefix over the tiles (32 keys x 32 tile
+//   count    each wavefront counts the keys of its tile of 512 entries in LDS
+//   scan     per key, the exclusive prefix over the tiles (16 keys x 64 tile
 //            segments per workgroup), and the key totals
 //   scatter  each workgroup scans the key totals, and each wavefront walks its
 //            tile in order, 64 entries at a time: an entry's place is its
 //            key's running count plus the lanes below it with the same key
 //            (found by one ballot per key bit)
 //
-// Bound by latency at these sizes (10^5-10^6 entries): a comparison merge sort
-// of 64-bit keys took 170-250 us in 15 launches where this takes about 20.
+// A wavefront requests its tile's entries before it uses the first (a tile of
+// 1,024 that loaded 64 at a time took a memory latency for each).
+//
+// Bound by latency at these sizes (10^5-10^6 entries).  The action rows of 96
+// positions (622,000 entries): a comparison merge sort of 64-bit keys 200 us in
+// 15 launches, these three 32 us (count 5.7, scan 13.5, scatter 12.9; with the
+// tiles of 1,024: 11 + 9 + 21).
 #include "common.hpp"
 
 namespace mantis {
 namespace {
 
 constexpr int kMaxKeys = 2048;
-constexpr int kTile = 1024;  // entries of a wavefront
+constexpr int kTile = 512;  // entries of a wavefront
+constexpr int kSteps = kTile / 64;
 constexpr int kWaves = 4;
 
 __global__ void __launch_bounds__(64 * kWaves)
@@ -29,21 +35,24 @@ class_count_kernel(const int64_t* __restrict__ key, int64_t n, int n_keys, int64
   for (int k = threadIdx.x; k < kWaves * kMaxKeys; k += 64 * kWaves) count[k / kMaxKeys][k % kMaxKeys] = 0;
   __syncthreads();
   const int64_t tile = int64_t(blockIdx.x) * kWaves + wave;
-#pragma unroll 4
-  for (int i = 0; i < kTile / 64; ++i) {
+  int64_t k[kSteps];
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) {  // (n > 0: a grid of no tiles is not launched)
     const int64_t e = tile * kTile + i * 64 + lane;
-    if (e < n) {
-      const int64_t k = key[e];
-      if (k >= 0 && k < n_keys) atomicAdd(&count[wave][k], 1);
-      else raise_flag(flag, MANTIS_FLAG_INDEX);
-    }
+    k[i] = key[e < n ? e : n - 1];
+  }
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) {
+    if (tile * kTile + i * 64 + lane >= n) continue;
+    if (k[i] >= 0 && k[i] < n_keys) atomicAdd(&count[wave][k[i]], 1);
+    else raise_flag(flag, MANTIS_FLAG_INDEX);
   }
   __syncthreads();
   if (tile < n_tiles)
     for (int k = lane; k < n_keys; k += 64) hist[tile * n_keys + k] = count[wave][k];
 }
 
-constexpr int kScanKeys = 32, kScanSegs = 32;
+constexpr int kScanKeys = 16, kScanSegs = 64;
 __global__ void __launch_bounds__(kScanKeys * kScanSegs)
 class_scan_kernel(int32_t* __restrict__ hist, int n_keys, int64_t n_tiles, int32_t* __restrict__ total) {
   __shared__ int32_t part[kScanSegs][kScanKeys + 1];
@@ -59,13 +68,20 @@ class_scan_kernel(int32_t* __restrict__ hist, int n_keys, int64_t n_tiles, int32
   part[seg][kk] = sum;
   __syncthreads();
   int32_t run = 0;
+#pragma unroll 8
   for (int s = 0; s < seg; ++s) run += part[s][kk];
   if (k >= n_keys) return;
   if (seg == kScanSegs - 1) total[k] = run + sum;
-  for (int64_t t = t0; t < t1; ++t) {
-    const int32_t c = hist[t * n_keys + k];
-    hist[t * n_keys + k] = run;
-    run += c;
+  constexpr int kAhead = 8;  // counts read before the first of them is overwritten
+  for (int64_t t = t0; t < t1; t += kAhead) {
+    int32_t c[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) c[u] = hist[(t + u < t1 ? t + u : t1 - 1) * n_keys + k];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (t + u < t1) hist[(t + u) * n_keys + k] = run;
+      run += c[u];
+    }
   }
 }
 
@@ -78,6 +94,14 @@ class_scatter_kernel(const int64_t* __restrict__ key, const int64_t* __restrict_
   __shared__ int32_t next[kWaves][kMaxKeys];
   __shared__ int32_t wave_sum[kWaves];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int64_t tile = int64_t(blockIdx.x) * kWaves + wave;
+  int64_t k64[kSteps], v[kSteps];
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) {
+    const int64_t e = tile * kTile + i * 64 + lane;
+    k64[i] = e < n ? key[e] : -1;
+    v[i] = e < n ? (col ? col[e] : e) : 0;
+  }
   // exclusive scan of the key totals: thread t owns keys kPer t ..
   int32_t c[kPer], own = 0;
 #pragma unroll
@@ -106,17 +130,15 @@ class_scatter_kernel(const int64_t* __restrict__ key, const int64_t* __restrict_
     for (int k = threadIdx.x; k < n_keys; k += 64 * kWaves) ptr[k] = start[k];
     if (threadIdx.x == 64 * kWaves - 1) ptr[n_keys] = run;  // the last thread's running sum: all entries
   }
-  const int64_t tile = int64_t(blockIdx.x) * kWaves + wave;
   if (tile >= n_tiles) return;  // (no barrier below)
   int32_t* mine = next[wave];
   for (int k = lane; k < n_keys; k += 64) mine[k] = start[k] + hist[tile * n_keys + k];
-  for (int i = 0; i < kTile / 64; ++i) {
-    const int64_t e = tile * kTile + i * 64 + lane;
-    if (tile * kTile + i * 64 >= n) break;  // uniform
-    const int64_t k64 = e < n ? key[e] : -1;
-    const int64_t v = e < n ? (col ? col[e] : e) : 0;
-    const bool ok = k64 >= 0 && k64 < n_keys;
-    const int k = ok ? int(k64) : 0;
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) {
+    // other lanes' counts: keep the reads of this step after the writes before it
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const bool ok = k64[i] >= 0 && k64[i] < n_keys;
+    const int k = ok ? int(k64[i]) : 0;
     uint64_t same = __ballot(ok);
     for (int b = 0; b < bits; ++b) {
       const uint64_t set = __ballot((k >> b) & 1);
@@ -127,7 +149,7 @@ class_scatter_kernel(const int64_t* __restrict__ key, const int64_t* __restrict_
       const int32_t at = mine[k] + below;
       // every lane of the key has read the count (one wavefront, LDS in order)
       if (below == 0) mine[k] = at + __popcll(same);
-      out[at] = v;
+      out[at] = v[i];
     }
   }
 }

@@ -281,10 +281,10 @@ def test_class_reduce_run_lengths(device, h, dt):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,n_keys", [(0, 5), (1, 1), (63, 2), (1024, 726), (1025, 729), (4097, 1458),
+@pytest.mark.parametrize("n,n_keys", [(0, 5), (1, 1), (63, 2), (512, 726), (513, 729), (4097, 1458),
                                       (70001, 2048), (3000, 2049)])
 def test_class_order(device, n, n_keys):
-    """Around the 1,024-entry tiles and the 2,048-key limit, one key owning
+    """Around the 512-entry tiles and the 2,048-key limit, one key owning
     half the entries: the stable argsort and its CSR."""
     gen = torch.Generator().manual_seed(15 + n)
     key = torch.where(torch.rand(n, generator=gen) < 0.5, n_keys // 2, torch.randint(0, n_keys, (n,), generator=gen))
