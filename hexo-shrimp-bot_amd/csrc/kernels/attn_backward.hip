@@ -268,15 +268,18 @@ attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_
 // dscore[E], E = cedge[j] (a query-major edge), and with kV partial[s] = sum
 // of alpha[E, head] * go[qid[E]].  dscore = alpha (dalpha - delta[qid]), or
 // with qid null dalpha_e already holds it.  16 entries per index load; the gradient
-// rows of kLook entries in flight, the scores one entry per lane.  Bound by
-// the gathered gradient rows.
+// rows of kLook entries in flight from clamped indices (a load under a
+// condition is waited for before the next), the scores one entry per lane.
+// Bound by the latency of the gathered gradient rows: with eight rows in
+// flight 147 and 53.5 us for 1,075,000 and 416,000 entries (four conditional
+// ones: 156 and 55.6), 22 and 19 for 193,000 and 74,000 (33 and 31).
 template <bool kV>
 __global__ void __launch_bounds__(kBlock)
 class_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ dalpha_e,
                    const float* __restrict__ delta, const float* __restrict__ go, int64_t ldgo, const int64_t* __restrict__ qid, int64_t n_q,
                    const int64_t* __restrict__ cedge, int64_t n_edges, const int64_t* __restrict__ slice_edge,
                    int64_t n_slices, float* __restrict__ partial, float* __restrict__ partial4, int32_t* flag) {
-  constexpr int kLook = 4;
+  constexpr int kLook = 8;
   const int64_t s = int64_t(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
   const int lane = threadIdx.x % kGroup;
   if (s >= n_slices) return;
@@ -308,22 +311,21 @@ class_slice_kernel(const float* __restrict__ alpha_e, const float* __restrict__ 
     }
     if constexpr (kV) {
       const int64_t row = ok ? qi : -1;
-      for (int j = 0; j < cnt; j += kLook) {
-        float gv[kLook][8], al[kLook];
+      for (int j = 0; j < cnt && n_q > 0; j += kLook) {
+        Chunk8<float> gv[kLook];
+        float al[kLook];
         bool use[kLook];
 #pragma unroll
-        for (int u = 0; u < kLook; ++u) {
+        for (int u = 0; u < kLook; ++u) {  // (an entry out of range reads row 0 and edge 0)
           const int from = j + u < cnt ? j + u : cnt - 1;
           const int64_t r = __shfl(row, from, kGroup), e = __shfl(E, from, kGroup);
           use[u] = j + u < cnt && r >= 0;
-          if (use[u]) {  // uniform over the group
-            load8(go + r * ldgo + c0, gv[u]);
-            al[u] = alpha_e[e * kHeads + h];
-          }
+          gv[u].load(go + (r >= 0 ? r : 0) * ldgo + c0);
+          al[u] = alpha_e[(r >= 0 ? e : 0) * kHeads + h];
         }
 #pragma unroll
         for (int u = 0; u < kLook; ++u)
-          if (use[u])
+          if (use[u])  // uniform over the group
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[i] = fmaf(al[u], gv[u][i], acc[i]);
       }
