@@ -309,29 +309,45 @@ latent_broadcast_bwd_kernel(LatArgs a) {
 
 // ---------------------------------------------------------------- finish
 
-// Blocks [0, n_pos): the splits' partial sums of a position's latent rows.
+// Blocks [0, n_pos * kParts): the splits' partial sums of a position's latent
+// rows, a column per thread and kAhead splits in flight, added in split order
+// (one workgroup per position, a split after the other, was 21 and 11.6 us of
+// a launch at 128 positions of 21 splits).
 // The others: 256 windows each, which the first launch has written if the
 // layout is window_latent_layout's; a window that its position's run of the
 // order does not name (mark holds no entry of that run naming it) gets its
 // rows here, from its own position.
+template <bool kRead>
+constexpr int kPartialWidth = (kRead ? 1 : 2) * kSlots * kRow;
+template <bool kRead>
+constexpr int kParts = kPartialWidth<kRead> / kBlock;
+constexpr int kAhead = 8;
 template <typename T, bool kRead>
 __global__ void __launch_bounds__(kBlock)
 latent_bwd_finish_kernel(LatArgs a) {
-  constexpr int kWidth = (kRead ? 1 : 2) * kSlots * kRow;
-  if (int64_t(blockIdx.x) < a.n_pos) {
-    const int64_t p = blockIdx.x;
-    for (int c = threadIdx.x; c < kWidth; c += kBlock) {
-      float x = 0.f;
-      for (int s = 0; s < a.splits; ++s) x += a.partial[(p * a.splits + s) * kWidth + c];
-      // dq or dk: times the score scale; dv: as summed
-      const bool second = c >= kSlots * kRow;
-      T* to = static_cast<T*>(kRead ? a.dq : second ? a.dv : a.dk);
-      from_f32(to[p * kSlots * kRow + c % (kSlots * kRow)], second ? x : x * a.scale);
+  constexpr int kWidth = kPartialWidth<kRead>;
+  const int64_t n_sums = a.n_pos * kParts<kRead>;
+  if (int64_t(blockIdx.x) < n_sums) {
+    const int64_t p = blockIdx.x / kParts<kRead>;
+    const int c = int(blockIdx.x % kParts<kRead>) * kBlock + threadIdx.x;
+    const float* from = a.partial + p * a.splits * kWidth + c;
+    float x = 0.f;
+    for (int s = 0; s < a.splits; s += kAhead) {
+      float y[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) y[u] = from[int64_t(s + u < a.splits ? s + u : a.splits - 1) * kWidth];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (s + u < a.splits) x += y[u];
     }
+    // dq or dk: times the score scale; dv: as summed
+    const bool second = c >= kSlots * kRow;
+    T* to = static_cast<T*>(kRead ? a.dq : second ? a.dv : a.dk);
+    from_f32(to[p * kSlots * kRow + c % (kSlots * kRow)], second ? x : x * a.scale);
     return;
   }
   const int lane = threadIdx.x % kGroup;
-  const int64_t first = (int64_t(blockIdx.x) - a.n_pos) * kBlock + threadIdx.x / kGroup * kGroup;
+  const int64_t first = (int64_t(blockIdx.x) - n_sums) * kBlock + threadIdx.x / kGroup * kGroup;
   const int64_t mine = first + lane;
   bool miss = false;
   if (mine < a.n_w) {
@@ -404,7 +420,7 @@ int32_t backward(LatArgs a, int32_t dtype, void* workspace, int64_t workspace_by
     if (p && !aligned16(p)) return MANTIS_E_ARG;
   if (!workspace || !aligned16(workspace) || workspace_bytes < partial_bytes(lat, win) + win * 4) return MANTIS_E_ARG;
   a.splits = int32_t(n_splits(lat, win));
-  const int64_t grid = lat * a.splits, finish = lat + (win + kBlock - 1) / kBlock;
+  const int64_t grid = lat * a.splits, finish = lat * kParts<kRead> + (win + kBlock - 1) / kBlock;
   if (grid > 2147483647LL || finish > 2147483647LL) return MANTIS_E_ARG;
   a.mark = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + partial_bytes(lat, win));
   a.scale = 0.17677669529663687f;  // 1 / sqrt(32)
