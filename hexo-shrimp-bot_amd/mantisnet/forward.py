@@ -1179,18 +1179,15 @@ def _cell_heads(model, w, g, cells, b: Batch, plan: Plan, mass_floor: float, raw
     return policy, q_score, q_values
 
 
-# The production configuration's evaluation runs as one native call that
-# queues its launches over one workspace (True, the default), or launch by
-# launch from here (False).  The native call takes the host 0.3 ms instead of
-# 1.7-1.9, which is the whole evaluation below about 60 positions; a traced
-# evaluation (ops.trace times each launch) and every other configuration or
-# batch form run launch by launch.
-NATIVE_LEAF = True
-
-
 def _leaf_of(model, b: Batch, dev) -> _hip_api.MantisLeafBatch | None:
+    """The batch for the native evaluation, or None where the evaluation runs
+    launch by launch from here: the production configuration's runs as one
+    native call that queues its launches over one workspace.  That takes the
+    host 0.3 ms instead of 1.7-1.9, which is the whole evaluation below about
+    60 positions.  A traced evaluation (ops.trace times each launch) and every
+    other configuration or batch form run launch by launch."""
     cfg = model.cfg
-    if not (NATIVE_LEAF and cfg.cell_nodes and cfg.cell_node_scope == "all" and cfg.blocks >= 1
+    if not (cfg.cell_nodes and cfg.cell_node_scope == "all" and cfg.blocks >= 1
             and cfg.value_hidden == 128 and cfg.value_bins <= 128 and FUSE_WINDOW_PROJECTION):
         return None
     if cfg.cell_structure or cfg.cell_adjacency or cfg.action_tactical or SPLIT_CELL_STAGES or ops.tracing_any():

@@ -324,7 +324,7 @@ def test_weights_changed_between_evaluations_are_used(device):
 
 
 @pytest.mark.parametrize("config,count", [(1, 1), (4, 1), (4, 9), (5, 2)])
-def test_native_leaf_is_bitwise_the_launch_by_launch_evaluation(device, config, count):
+def test_native_leaf_is_bitwise_the_launch_by_launch_evaluation(device, config, count, monkeypatch):
     # one native call over one workspace against the same launches queued from
     # Python: every output of the forward, and the evaluator's head rows
     from mantisnet import forward, ops
@@ -332,18 +332,15 @@ def test_native_leaf_is_bitwise_the_launch_by_launch_evaluation(device, config, 
     net = _model(device, PRODUCTION, seed=6)
     batch = collate_positions(synthetic.random_games(config, count, start=700)).to(device)
     outs = []
-    saved = forward.NATIVE_LEAF
-    try:
-        for native in (True, False):
-            forward.NATIVE_LEAF = native
-            assert (forward._leaf_of(net, batch, batch.stone_own.device) is not None) == native
-            with torch.no_grad():
-                out = net(batch, 0.2)
-                outs.append([getattr(out, n) for n in ("policy_logits", "q_score", "q_values", "value", "value_dist",
-                                                       "value_logits")] + list(forward.policy_q(net, batch)))
-            ops.raise_on_device_error(device)
-    finally:
-        forward.NATIVE_LEAF = saved
+    assert forward._leaf_of(net, batch, batch.stone_own.device) is not None
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(forward, "_leaf_of", lambda *_: None)
+        with torch.no_grad():
+            out = net(batch, 0.2)
+            outs.append([getattr(out, n) for n in ("policy_logits", "q_score", "q_values", "value", "value_dist",
+                                                   "value_logits")] + list(forward.policy_q(net, batch)))
+        ops.raise_on_device_error(device)
     for a, b in zip(*outs):
         assert a.shape == b.shape and torch.equal(a, b)
 
