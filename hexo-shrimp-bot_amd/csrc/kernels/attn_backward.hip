@@ -52,23 +52,40 @@ struct AttnBwd {
   const float* m;  // (n_q, 4)
   const float* l;  // (n_q, 4)
   float* delta;    // (n_q, 4)
+  float4* stats;   // (n_q, 4): m, 1 / l (0 for a row without entries), delta
   float scale;
   int32_t* flag;
 };
 
+// x, or zeros: a row that is not to count must not bring its infinities in
+template <typename T>
+__device__ __forceinline__ void keep(Chunk8<T>& x, bool ok) {
+  if constexpr (std::is_same_v<T, float>) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x.f[i] = ok ? x.f[i] : 0.f;
+  } else {
+    x.u.x = ok ? x.u.x : 0u, x.u.y = ok ? x.u.y : 0u, x.u.z = ok ? x.u.z : 0u, x.u.w = ok ? x.u.w : 0u;
+  }
+}
+
 // Query-major pass: 16 lanes per query row; up to 16 of its entries are loaded
 // at once, one per lane, and shared by shuffles, so the rows of kB entries are
-// in flight together (an entry at a time, each waited for its own chain of
-// index and rows).  Bound by the gathered rows.  With alpha_e, alpha and
-// dalpha of every entry are kept for the class sums; with finish the lane that
-// wrote them turns dalpha into dscore (callers without qid, whose class pass
-// cannot look delta up).
+// in flight together and their score chains (two head sums and an exponential)
+// run side by side.  Bound by the chain pointers -> indices -> rows and the
+// rows in flight: two entries per step, so that four wavefronts fit a SIMD
+// (64 positions, bf16, 1,075,000 / 416,000 / 416,000 entries: 138 / 112 / 43
+// us; four entries and a branch per entry 144 / 114 / 42; four side by side,
+// three wavefronts, 143 / 113 / 51; without the q and gradient rows of queries
+// that have no entry 144 / 114 / 43).  With alpha_e, alpha and dalpha of every
+// entry are kept for the class sums; with finish the lane that wrote them
+// turns dalpha into dscore (callers without qid, whose class pass cannot look
+// delta up).
 template <typename T, typename Tv, bool kVcls>
 __global__ void __launch_bounds__(kBlock)
 attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t* __restrict__ src,
                   const int64_t* __restrict__ cls, int64_t n_entries, T* __restrict__ dq,
                   float* __restrict__ alpha_e, float* __restrict__ dalpha_e, bool finish) {
-  constexpr int kB = sizeof(T) == 2 ? 4 : 2;
+  constexpr int kB = 2;
   const int64_t row = int64_t(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
   const int lane = threadIdx.x % kGroup;
   if (row >= a.n_q) return;
@@ -84,6 +101,7 @@ attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t*
   load8(a.go + row * a.ldgo + c0, gv);
   const float mm = a.m[row * kHeads + h], ll = a.l[row * kHeads + h];
   const float inv = ll > 0.f ? 1.f / ll : 0.f;
+  const float* bias = a.bias + h * a.n_classes;  // (read only if a.bias)
   float A[8] = {0, 0, 0, 0, 0, 0, 0, 0}, B[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   float delta = 0.f;
   for (int64_t base = st; base < en; base += kGroup) {
@@ -92,53 +110,62 @@ attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t*
     const int64_t s = src[mine], c = cls ? cls[mine] : 0;
     const bool good = s >= 0 && s < a.n_k && c >= 0 && (!cls || c < a.n_classes);
     if (!good && lane < cnt) raise_flag(a.flag, MANTIS_FLAG_INDEX);
-    const int64_t s_ok = good ? s : 0;
-    const int32_t c_ok = good ? int32_t(c) : 0;
+    const int32_t c_in = good ? int32_t(c) : -1;
+    // the entry's row offsets once, by its lane: 64-bit products are 16 cycles each
+    const int64_t k_at = good ? s * a.ldk : 0, v_at = good ? s * a.ldv : 0;
+    if (a.n_k <= 0) {  // no row to read: every entry is flagged
+      if (alpha_e && (lane & 3) == 0)
+        for (int64_t e = base; e < base + cnt; ++e) alpha_e[e * kHeads + h] = dalpha_e[e * kHeads + h] = 0.f;
+      continue;
+    }
     for (int j = 0; j < cnt; j += kB) {
       Chunk8<T> xk[kB], xv[kB];
       Chunk8<Tv> xc[kB];
-      float bs[kB];
+      float bs[kB], sd[kB], dd[kB];
       bool ok[kB];
 #pragma unroll
-      for (int u = 0; u < kB; ++u) {
+      for (int u = 0; u < kB; ++u) {  // (an entry that is not ok reads row 0)
         const int from = j + u < cnt ? j + u : cnt - 1;
-        const int64_t su = __shfl(s_ok, from, kGroup);
-        const int32_t cu = __shfl(c_ok, from, kGroup);
-        ok[u] = __shfl(int(good), from, kGroup) != 0 && j + u < cnt;
-        if (a.n_k > 0) {  // (an entry that is not ok reads row 0)
-          xk[u].load(kb + su * a.ldk);
-          xv[u].load(vb + su * a.ldv);
-        }
-        if constexpr (kVcls) xc[u].load(cb + int64_t(cu) * kRow);
-        bs[u] = a.bias ? a.bias[h * a.n_classes + cu] : 0.f;
+        const int32_t cu = __shfl(c_in, from, kGroup);
+        ok[u] = cu >= 0 && j + u < cnt;
+        xk[u].load(kb + __shfl(k_at, from, kGroup));
+        xv[u].load(vb + __shfl(v_at, from, kGroup));
+        const uint32_t co = cu < 0 ? 0u : uint32_t(cu);
+        if constexpr (kVcls) xc[u].load(cb + int64_t(co) * kRow);
+        bs[u] = a.bias ? bias[co] : 0.f;
       }
+      // without a branch between them the entries' chains run side by side
 #pragma unroll
       for (int u = 0; u < kB; ++u) {
-        const int64_t e = base + j + u;
-        if (!ok[u]) {  // uniform over the group
-          if (j + u < cnt && alpha_e && (lane & 3) == 0) alpha_e[e * kHeads + h] = dalpha_e[e * kHeads + h] = 0.f;
-          continue;
-        }
-        float sd = 0.f, dd = 0.f;
+        sd[u] = dd[u] = 0.f;
+        keep(xk[u], ok[u]);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           float vv = xv[u][i];
           if constexpr (kVcls) vv += xc[u][i];
-          sd = fmaf(qv[i], xk[u][i], sd);
-          dd = fmaf(gv[i], vv, dd);
+          sd[u] = fmaf(qv[i], xk[u][i], sd[u]);
+          dd[u] = fmaf(gv[i], vv, dd[u]);
         }
-        sd = head_sum(sd);
-        dd = head_sum(dd);
-        const float al = expf(sd * a.scale + bs[u] - mm) * inv;
-        delta = fmaf(al, dd, delta);
+      }
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        sd[u] = head_sum(sd[u]);
+        dd[u] = head_sum(dd[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const float al = ok[u] ? expf(sd[u] * a.scale + bs[u] - mm) * inv : 0.f;
+        const float da = ok[u] ? dd[u] : 0.f, ad = al * da;
+        delta = fmaf(al, da, delta);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          A[i] = fmaf(al * dd, xk[u][i], A[i]);
+          A[i] = fmaf(ad, xk[u][i], A[i]);
           B[i] = fmaf(al, xk[u][i], B[i]);
         }
-        if (alpha_e && (lane & 3) == 0) {
+        if (alpha_e && (lane & 3) == 0 && j + u < cnt) {
+          const int64_t e = base + j + u;
           alpha_e[e * kHeads + h] = al;
-          dalpha_e[e * kHeads + h] = dd;
+          dalpha_e[e * kHeads + h] = da;
         }
       }
     }
@@ -149,6 +176,7 @@ attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t*
   store8(dq + row * kRow + c0, d);
   if ((lane & 3) == 0) {
     a.delta[row * kHeads + h] = delta;
+    a.stats[row * kHeads + h] = make_float4(mm, inv, delta, 0.f);
     // this lane wrote these entries above: dscore = alpha (dalpha - delta)
     if (finish)
       for (int64_t e = st; e < en; ++e)
@@ -161,6 +189,9 @@ attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t*
 // runs (windows and cells: about five entries); a stone's run of 200 radius
 // entries left 5,000 groups each walking its own chain, a quarter of a
 // launch's lanes, so long runs get 4 groups (a wavefront) or 16 (a workgroup).
+// The query pass leaves m, 1 / l and delta of a query's head side by side: one
+// 16-byte load per entry instead of three and no division (64 positions, bf16:
+// 118.6 / 54.8 -> 113.3 / 51 us; 80 for the pass without class values, as before).
 template <typename T, typename Tv, bool kVcls, int kG>
 __global__ void __launch_bounds__(kBlock)
 attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_t* __restrict__ sqid,
@@ -181,6 +212,7 @@ attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_
   float kv[8], vv[8];
   load8(static_cast<const T*>(a.k) + row * a.ldk + c0, kv);
   load8(static_cast<const T*>(a.v) + row * a.ldv + c0, vv);
+  const float* bias = a.bias + h * a.n_classes;  // (read only if a.bias)
   float gk[8] = {0, 0, 0, 0, 0, 0, 0, 0}, gvv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   for (int64_t base = st + int64_t(group % kG) * kGroup; base < en; base += kG * kGroup) {
     const int cnt = int(en - base < kGroup ? en - base : kGroup);
@@ -188,48 +220,53 @@ attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_
     const int64_t qi = sqid[mine], c = scls ? scls[mine] : 0;
     const bool good = qi >= 0 && qi < a.n_q && c >= 0 && (!scls || c < a.n_classes);
     if (!good && lane < cnt) raise_flag(a.flag, MANTIS_FLAG_INDEX);
-    const int64_t q_ok = good ? qi : 0;
-    const int32_t c_ok = good ? int32_t(c) : 0;
+    const int32_t c_in = good ? int32_t(c) : -1;
+    const int64_t q_in = good ? qi : 0, q_at = q_in * a.ldq, g_at = q_in * a.ldgo;
+    if (a.n_q <= 0) continue;  // no row to read: every entry is flagged
     for (int j = 0; j < cnt; j += kB) {
       Chunk8<T> xq[kB];
       Chunk8<float> xg[kB];
       Chunk8<Tv> xc[kB];
-      float bs[kB], ml[kB], ll[kB], dl[kB];
+      float4 st4[kB];
+      float bs[kB], sd[kB], dd[kB];
       bool ok[kB];
 #pragma unroll
-      for (int u = 0; u < kB; ++u) {
+      for (int u = 0; u < kB; ++u) {  // (an entry that is not ok reads row 0)
         const int from = j + u < cnt ? j + u : cnt - 1;
-        const int64_t qu = __shfl(q_ok, from, kGroup);
-        const int32_t cu = __shfl(c_ok, from, kGroup);
-        ok[u] = __shfl(int(good), from, kGroup) != 0 && j + u < cnt;
-        if (a.n_q > 0) {  // (an entry that is not ok reads row 0)
-          xq[u].load(qb + qu * a.ldq);
-          xg[u].load(gb + qu * a.ldgo);
-          ml[u] = a.m[qu * kHeads + h];
-          ll[u] = a.l[qu * kHeads + h];
-          dl[u] = a.delta[qu * kHeads + h];
-        }
-        if constexpr (kVcls) xc[u].load(cb + int64_t(cu) * kRow);
-        bs[u] = a.bias ? a.bias[h * a.n_classes + cu] : 0.f;
+        const int32_t cu = __shfl(c_in, from, kGroup);
+        ok[u] = cu >= 0 && j + u < cnt;
+        xq[u].load(qb + __shfl(q_at, from, kGroup));
+        xg[u].load(gb + __shfl(g_at, from, kGroup));
+        st4[u] = a.stats[__shfl(q_in, from, kGroup) * kHeads + h];
+        const uint32_t co = cu < 0 ? 0u : uint32_t(cu);
+        if constexpr (kVcls) xc[u].load(cb + int64_t(co) * kRow);
+        bs[u] = a.bias ? bias[co] : 0.f;
       }
 #pragma unroll
       for (int u = 0; u < kB; ++u) {
-        if (!ok[u]) continue;  // uniform over the group
-        float sd = 0.f, dd = 0.f;
+        sd[u] = dd[u] = 0.f;
+        keep(xq[u], ok[u]);
+        keep(xg[u], ok[u]);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           float ve = vv[i];
           if constexpr (kVcls) ve += xc[u][i];
-          sd = fmaf(xq[u][i], kv[i], sd);
-          dd = fmaf(xg[u][i], ve, dd);
+          sd[u] = fmaf(xq[u][i], kv[i], sd[u]);
+          dd[u] = fmaf(xg[u][i], ve, dd[u]);
         }
-        sd = head_sum(sd);
-        dd = head_sum(dd);
-        const float al = ll[u] > 0.f ? expf(sd * a.scale + bs[u] - ml[u]) / ll[u] : 0.f;
-        const float ds = al * (dd - dl[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        sd[u] = head_sum(sd[u]);
+        dd[u] = head_sum(dd[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const float al = ok[u] && st4[u].y > 0.f ? expf(sd[u] * a.scale + bs[u] - st4[u].x) * st4[u].y : 0.f;
+        const float ds = ok[u] ? al * (dd[u] - st4[u].z) * a.scale : 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          gk[i] = fmaf(ds * a.scale, xq[u][i], gk[i]);
+          gk[i] = fmaf(ds, xq[u][i], gk[i]);
           gvv[i] = fmaf(al, xg[u][i], gvv[i]);
         }
       }
@@ -397,17 +434,18 @@ bool with_type(int32_t dtype, F&& fn) {
   }
 }
 
-// Workspace of the attention backward: delta, per-edge alpha and dalpha,
+// Workspace of the attention backward: delta, the packed row terms, per-edge alpha and dalpha,
 // the class slice tables and the two kinds of partial rows.
 struct AttnLayout {
-  int64_t delta, alpha, dalpha, slices, total;
+  int64_t delta, stats, alpha, dalpha, slices, total;
 };
 
-// (untyped edges, n_classes == 0, need delta alone)
+// (untyped edges, n_classes == 0, need no per-edge terms)
 AttnLayout attn_layout(int64_t n_q, int64_t n_edges, int64_t n_classes) {
   AttnLayout L;
   L.delta = 0;
-  L.alpha = L.delta + align256(n_q * kHeads * 4);
+  L.stats = L.delta + align256(n_q * kHeads * 4);
+  L.alpha = L.stats + align256(n_q * kHeads * 16);
   if (n_classes == 0) {
     L.dalpha = L.slices = L.total = L.alpha;
     return L;
@@ -459,7 +497,7 @@ int32_t mantis_attention_backward(const void* q, const void* k, const void* v, i
   if (!workspace || workspace_bytes < L.total || !aligned16(workspace)) return MANTIS_E_ARG;
   char* ws = static_cast<char*>(workspace);
   AttnBwd a{q, k, v, ldq, ldk, ldv, n_q, n_k, bias, n_classes, vcls, grad_out, ldgo, m, l,
-            reinterpret_cast<float*>(ws + L.delta), 0.17677669529663687f, err_flag};
+            reinterpret_cast<float*>(ws + L.delta), reinterpret_cast<float4*>(ws + L.stats), 0.17677669529663687f, err_flag};
   // per-edge softmax terms: kept for the class sums of typed edges only
   float* alpha_e = typed ? reinterpret_cast<float*>(ws + L.alpha) : nullptr;
   float* dalpha_e = typed ? reinterpret_cast<float*>(ws + L.dalpha) : nullptr;
