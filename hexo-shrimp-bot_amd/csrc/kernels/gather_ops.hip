@@ -111,7 +111,7 @@ segment_order_kernel(const int64_t* __restrict__ seg_ptr, int64_t n_seg, const i
 
 // ------------------------------------------------------------ run reduction
 
-template <typename Tin, typename Tout>
+template <typename Tin, typename Tout, int kLook>
 __global__ void __launch_bounds__(kBlock)
 run_reduce_kernel(const Tin* __restrict__ values, int64_t n_src, int64_t ld, int64_t h,
                   const int64_t* __restrict__ gather, const int64_t* __restrict__ ptr,
@@ -122,16 +122,20 @@ run_reduce_kernel(const Tin* __restrict__ values, int64_t n_src, int64_t ld, int
   int64_t start, end;
   segment(ptr, row, n_entries, start, end);
   // Up to 16 of the run's source indices at once (one per lane, unconditional
-  // from a clamped slot), shared by shuffles; four source rows in flight.
-  // The sum runs over the entries in order, so it is the same fp32 sum as
-  // one entry at a time.
-  constexpr int kLook = 4;
+  // from a clamped slot), shared by shuffles; kLook source rows in flight: 4
+  // under their conditions (short runs; 64 registers of fp32 rows at 8), or 8
+  // unconditional 16-bit rows for long runs, which wait for each other less
+  // (16 stones of 18 windows, fp16: 9.5 -> 4.8 us per launch; three launches
+  // over fp32 rows at 96 positions: 58.9 us with 4, 61.6 with 8).  The sum
+  // runs over the entries in order, so it is the same fp32 sum as one entry at
+  // a time.
   // every lane runs every chunk step (the shuffles need all 16 lanes); a lane
   // past the row's width only skips its loads and its store
   // (128 columns per grid row: the chunks of a wide row run side by side)
   for (int64_t cb = int64_t(blockIdx.y) * (kGroup * 8); cb < h; cb += int64_t(gridDim.y) * (kGroup * 8)) {
     const int64_t c0 = cb + int64_t(lane) * 8;
     const bool mine = c0 < h;
+    const Tin* col = values + (mine ? c0 : 0);  // a lane past the width reads the first columns
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int64_t base = start; base < end; base += kGroup) {
       const int cnt = int(end - base < kGroup ? end - base : kGroup);
@@ -140,19 +144,20 @@ run_reduce_kernel(const Tin* __restrict__ values, int64_t n_src, int64_t ld, int
       const bool mine_ok = my >= 0 && my < n_src;
       if (lane < cnt && !mine_ok) raise_flag(flag, MANTIS_FLAG_INDEX);
       const int32_t my32 = mine_ok ? int32_t(my) : -1;  // n_src fits int32 (host check)
+      if (n_src <= 0) continue;  // no row to read: every entry is flagged
       for (int j = 0; j < cnt; j += kLook) {
-        float x[kLook][8];
+        Chunk8<Tin> x[kLook];
         bool ok[kLook];
 #pragma unroll
-        for (int u = 0; u < kLook; ++u) {
+        for (int u = 0; u < kLook; ++u) {  // (with kLook 8 an entry out of range reads row 0)
           const int idx = j + u < cnt ? j + u : cnt - 1;
           const int32_t src = __shfl(my32, idx, kGroup);
           ok[u] = j + u < cnt && src >= 0;
-          if (mine && ok[u]) load8(values + int64_t(src) * ld + c0, x[u]);
+          if (kLook == 8 || ok[u]) x[u].load(col + int64_t(src < 0 ? 0 : src) * ld);
         }
 #pragma unroll
         for (int u = 0; u < kLook; ++u)
-          if (mine && ok[u])
+          if (ok[u])  // uniform over the group
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[i] += x[u][i];
       }
@@ -867,11 +872,14 @@ int32_t mantis_run_reduce(const void* values, int32_t values_dtype, int64_t n_sr
                                                         (kGroupsPerBlock * kRowsRR))),
                                          block, 0, s>>>(static_cast<const TI*>(values), n_src, ld, gather, ptr,
                                                         n_dest, n_entries, static_cast<TO*>(out), err_flag);
-      else if (vec)
-        run_reduce_kernel<TI, TO><<<dim3(grid.x, unsigned(std::min<int64_t>((h + 127) / 128, 65535))), block, 0, s>>>(static_cast<const TI*>(values), n_src, ld,
-                                                         h, gather, ptr, n_dest, n_entries,
-                                                         static_cast<TO*>(out), err_flag);
-      else
+      else if (vec) {
+        // (the reason for either number of rows in flight is at the kernel)
+        const auto kernel = sizeof(TI) == 2 && n_entries >= 4 * n_dest ? run_reduce_kernel<TI, TO, 8>
+                                                                       : run_reduce_kernel<TI, TO, 4>;
+        const dim3 chunks(grid.x, unsigned(std::min<int64_t>((h + 127) / 128, 65535)));
+        kernel<<<chunks, block, 0, s>>>(static_cast<const TI*>(values), n_src, ld, h, gather, ptr, n_dest, n_entries,
+                                        static_cast<TO*>(out), err_flag);
+      } else
         run_reduce_scalar_kernel<TI, TO><<<grid, block, 0, s>>>(
             static_cast<const TI*>(values), n_src, ld, h, gather, ptr, n_dest, n_entries,
             static_cast<TO*>(out), err_flag);
