@@ -19,7 +19,7 @@
 // no atomics: two calls agree bitwise.
 //
 // (128 positions of 40-120 stones, 169k windows, bf16: forward and backward of
-// the read and the broadcast together 4,810 -> 365 us; before, each operator
+// the read and the broadcast together 4,810 -> 336 us; before, each operator
 // ran two passes of 1.1 ms over a materialised edge list.)
 #include "common.hpp"
 #include "gather.hpp"
