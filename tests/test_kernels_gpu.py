@@ -53,6 +53,37 @@ def test_run_reduce_matches_index_add(device, vdt, odt, h):
     torch.testing.assert_close(out.float().cpu(), exp, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("h,dt", [(8, torch.float16), (128, torch.bfloat16), (136, torch.float16),
+                                  (256, torch.float32)])
+def test_run_reduce_long_runs(device, h, dt):
+    """Runs of more than four entries on average around the 8 rows in flight
+    and the 16 indices of a load, empty runs, widths off the 128-column chunks;
+    an index out of range adds nothing and is flagged, with finite sums though
+    source row 0 is infinite."""
+    gen = torch.Generator().manual_seed(31)
+    lens = torch.tensor([0, 1, 7, 8, 9, 15, 16, 17, 24, 33, 0, 100])
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    values = torch.randn(50, h, generator=gen).to(dt)
+    values[0] = float("inf")
+    rows = torch.randint(1, 50, (int(lens.sum()),), generator=gen)
+    dest = torch.repeat_interleave(torch.arange(len(lens)), lens)
+
+    def ref(keep):
+        return torch.zeros(len(lens), h, dtype=torch.float64).index_add_(0, dest[keep], values.double()[rows[keep]])
+
+    got = ops.run_reduce(values.to(device), rows.to(device), ptr.to(device), len(lens), torch.float32)
+    ops.raise_on_device_error(device)
+    keep = torch.ones(len(rows), dtype=torch.bool)
+    # fp32 sums of up to 100 values near 1 in a row
+    torch.testing.assert_close(got.double().cpu(), ref(keep), rtol=1e-5, atol=1e-4)
+    rows[3], rows[-1] = 50, -1
+    keep[3] = keep[-1] = False
+    got = ops.run_reduce(values.to(device), rows.to(device), ptr.to(device), len(lens), torch.float32)
+    torch.testing.assert_close(got.double().cpu(), ref(keep), rtol=1e-5, atol=1e-4)
+    with pytest.raises(ValueError):
+        ops.raise_on_device_error(device)
+
+
 def test_out_of_range_index_is_flagged_not_read(device):
     dest = torch.tensor([0, 0, 1, 2])
     gather = torch.tensor([0, 5, 1, 2])  # 5 is out of range for 3 source rows
