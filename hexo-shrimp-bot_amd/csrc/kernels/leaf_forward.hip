@@ -237,7 +237,7 @@ value_tail_kernel(const float* __restrict__ read, int64_t n_pos, const float* __
     float s = b0[o];
 #pragma unroll
     for (int k = 0; k < kParts; ++k) s += part[k][g][o];
-    hid[g][o] = fmaxf(s, 0.f);
+    hid[g][o] = s < 0.f ? 0.f : s;  // (a NaN stays one: fmaxf would answer 0)
   }
   __syncthreads();
 #pragma unroll

@@ -383,6 +383,13 @@ def test_value_tail_and_latent_out_match_torch(device):
         torch.testing.assert_close(logits.cpu().double(), x, rtol=1e-5, atol=1e-5)
         torch.testing.assert_close(dist.cpu().double(), x.softmax(-1), rtol=1e-4, atol=1e-6)
         torch.testing.assert_close(value.cpu().double(), x.softmax(-1) @ bins.double(), rtol=1e-4, atol=1e-5)
+        # a NaN in one position's read: that position's outputs only, the
+        # other positions of its workgroup as before
+        read[p // 2, 7] = float("nan")
+        bad = ops.value_tail(d(read), d(w0.t().contiguous()), d(b0), d(w2.t().contiguous()), d(b2), d(bins))
+        for a, b in zip(bad, (value, dist, logits)):
+            keep = torch.arange(p) != p // 2
+            assert torch.isnan(a[p // 2]).all() and torch.equal(a.cpu()[keep], b.cpu()[keep])
         out, half = ops.latent_out(d(g), d(gamma), d(beta), d(glin.t().contiguous()))
         exp = torch.nn.functional.layer_norm(g.double(), (128,), gamma.double(), beta.double(), 1e-5).view(p, 4, 128).mean(1)
         torch.testing.assert_close(out.cpu().double(), exp, rtol=1e-5, atol=1e-5)
