@@ -564,17 +564,28 @@ int32_t launch(const Args& a, hipStream_t stream, int columns = 1) {
   return launched();
 }
 
+// Whether the output rows' bytes can touch the input rows'.
+template <typename TX>
+bool rows_overlap(const Args& a, int64_t n1) {
+  const char* x = static_cast<const char*>(a.x);
+  const char* o = static_cast<const char*>(a.out);
+  return x < o + ((a.m - 1) * a.ldo + n1) * 2 && o < x + ((a.n_x - 1) * a.ldx + kK) * int64_t(sizeof(TX));
+}
+
 // A LayerNorm'd projection to fp16 rows, n1 wide (a multiple of 128).  A
 // workgroup stages all the weights of its columns before its first row (64 KB
 // for 256 columns, 128 KB for 512), which is most of a launch over a few
 // hundred rows, so a launch that leaves CUs idle cuts its columns over grid
 // rows of 64 or 128 as long as every workgroup then has a CU of its own.  Each
 // output is computed as before.  (512 wide over the four latent rows of one
-// position: 13.3 us uncut, 4.6 cut; 2,048 rows 17.8 and 6.2.)
+// position: 13.3 us uncut, 4.6 cut; 2,048 rows 17.8 and 6.2.)  Uncut, the
+// wavefront that reads a row is the only one that writes it, so the output may
+// lie over the input; cut, one workgroup would store over a row that another
+// has still to read, so such a launch stays whole.
 template <typename TX, int N1>
 int32_t launch_columns(const Args& a, hipStream_t s) {
   const int64_t tiles = (a.m + 127) / 128;  // rows of a 512-thread workgroup
-  const int64_t cus = cu_count();
+  const int64_t cus = rows_overlap<TX>(a, N1) ? 0 : cu_count();
   if (tiles * (N1 / 64) <= cus) return launch<TX, float, true, 64, false, false, false, 0, false, true>(a, s, N1 / 64);
   if (N1 > 128 && tiles * (N1 / 128) <= cus)
     return launch<TX, float, true, 128, false, false, false, 0, false, true>(a, s, N1 / 128);

@@ -877,6 +877,9 @@ int64_t mantis_stone_attention_schedule_len(int64_t n_pos, int32_t heads, int64_
  * rows, fp16 out), the residual projection (n1 = 128, fp32 or fp16 residual), the
  * two-layer residual MLPs (n1 = 128 with x2 into fp32 or fp16 residual rows,
  * n1 = 256 without) and the two-layer head (n1 = 256 with x2, fp32 out).
+ * Without x_rows, out_mode 0's out may lie over x where each output row's
+ * bytes meet only the bytes of its own input row (out == x, or x the first
+ * columns of out's rows).
  */
 int32_t mantis_fused_linear(const void* x, int32_t x_dtype, int64_t ldx, const int64_t* x_rows,
                             int64_t n_x, int64_t m, int32_t layer_norm, const void* x2,

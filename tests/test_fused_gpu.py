@@ -952,6 +952,33 @@ def test_few_row_projections_cut_by_columns_are_bitwise_the_whole(device, n1, dt
         assert torch.equal(ops.fused_linear(x, w, b, layer_norm=True, x_rows=rows), whole[:m].flip(0))
 
 
+@pytest.mark.parametrize("m", [1, 130, 4100])
+def test_few_row_projections_into_their_own_rows(device, m):
+    # rows that a launch could cut by columns, written where they are read: in
+    # place, as the upper columns of a buffer whose first columns they are, over
+    # the first half of the fp32 rows, and beside them in one buffer
+    gen = _g(19)
+    x32 = torch.randn(m, 128, generator=gen).to(device)
+    x = x32.to(H16)
+    w = (torch.randn(256, 128, generator=gen) / 11).to(H16).to(device)
+    b = torch.randn(256, generator=gen).to(device)
+
+    def run(x, n1, out=None):
+        return ops.fused_linear(x, w[:n1], b[:n1], layer_norm=True, out=out)
+
+    for n1 in (128, 256):
+        exp, exp32 = run(x, n1), run(x32, n1)
+        wide = torch.zeros(m, 512, dtype=H16, device=device)
+        wide[:, :128] = x
+        assert torch.equal(run(wide[:, :128], n1, out=wide[:, :n1]), exp)
+        wide[:, :128] = x
+        assert torch.equal(run(wide[:, :128], n1, out=wide[:, 128:128 + n1]), exp)
+        assert torch.equal(wide[:, :128], x)
+        rows = x32.clone()
+        assert torch.equal(run(rows, n1, out=rows.view(H16)[:, :n1]), exp32)
+    assert torch.equal(run(x, 128, out=x), run(x32.to(H16), 128))
+
+
 def test_latent_mix_over_more_positions_than_workgroups(device):
     # 1,100 positions (1,024 workgroups at most): each as in a launch of its own
     gen = _g(18)
