@@ -102,14 +102,19 @@ class Prepared:
         # True while the last check found the parameters unchanged: the next
         # evaluation may then run before its check (see _speculative)
         self.steady = False
-        self._leaf = None  # (struct, its blocks, the tensors they point into)
+        self._leaf = None  # (the operands it was packed from, the pack)
 
     def leaf(self):
         """The operands as mantis_leaf_forward takes them, packed once per
-        rebuild; the pack holds every tensor it points into."""
-        if self._leaf is None:
-            self._leaf = _pack_leaf(self.model.cfg, self.t, self.params)
-        return self._leaf[0]
+        rebuild: (struct, its blocks, every tensor they point into).  The
+        caller holds the pack for as long as the call runs: another thread's
+        evaluation may find the parameters changed and replace it meanwhile
+        (the call runs without the interpreter lock), and a pack of operands
+        that were replaced while it was built serves its own call only."""
+        t, kept = self.t, self._leaf
+        if kept is None or kept[0] is not t:
+            kept = self._leaf = t, _pack_leaf(self.model.cfg, t, self.params)
+        return kept[1]
 
     def refresh(self):
         # the module's parameter set is fixed after construction; what changes
@@ -128,7 +133,6 @@ class Prepared:
             with torch.no_grad():
                 self.t = _prepare(self.model, {n: p.detach().float() for n, p in self.params.items()})
             self.key = key
-            self._leaf = None
         self.steady = not changed
         return changed
 
@@ -1250,7 +1254,8 @@ def forward(model, batch: Batch, mass_floor: float):
         return policy, q_score, q_values, value, value_dist, value_logits
 
     def native(leaf, W):
-        return ops.leaf_forward(W.leaf(), leaf, model.bin_centers, mass_floor, dev)
+        pack = W.leaf()  # (held until the call returns)
+        return ops.leaf_forward(pack[0], leaf, model.bin_centers, mass_floor, dev)
 
     return _speculative(model, b, evaluate, native)
 
@@ -1270,7 +1275,8 @@ def policy_q(model, batch: Batch):
         return _head_rows(model, w, g, c, b, plan, raw_cells=True, W=W, g_half=half[0])
 
     def native(leaf, W):
-        return ops.leaf_forward(W.leaf(), leaf, None, 0.0, dev)
+        pack = W.leaf()  # (held until the call returns)
+        return ops.leaf_forward(pack[0], leaf, None, 0.0, dev)
 
     rows = _speculative(model, b, evaluate, native)
     return rows[:, 0].contiguous(), rows[:, 1:4]
