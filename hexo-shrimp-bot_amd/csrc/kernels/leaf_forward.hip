@@ -10,6 +10,7 @@
 // (prefix_*_kernel), the latent output with the heads' position half
 // (latent_out_kernel) and the value MLP (value_tail_kernel), all fp32.
 #include <algorithm>
+#include <initializer_list>
 
 #include "common.hpp"
 
@@ -380,6 +381,54 @@ bool sizes_ok(const mantis_leaf_batch& b) {
   return b.max_t >= 4 && b.max_t <= 2048 && b.n_pos * b.max_t <= 2147483647LL;
 }
 
+using Ptrs = std::initializer_list<const void*>;
+bool all_set(Ptrs ps) { return std::all_of(ps.begin(), ps.end(), [](const void* p) { return p != nullptr; }); }
+bool all_aligned(Ptrs ps) { return std::all_of(ps.begin(), ps.end(), [](const void* p) { return aligned16(p); }); }
+
+// What the launches below read without a check of their own, and what the
+// entry points they call would refuse once launches before them are queued.
+// (The biases of the row projections may be null, as those entries take them.)
+bool batch_ok(const mantis_leaf_batch& b) {
+  return all_set({b.stone_own, b.window_feat, b.moves_idx, b.inc_stone, b.inc_window, b.inc_class, b.stone_slot,
+                  b.window_slot, b.legal_offsets, b.cell_pos, b.cell_nearest, b.radius_src, b.radius_dst,
+                  b.radius_orbit, b.radius_own, b.radius_on_axis, b.dec_cell, b.dec_window, b.dec_class, b.act_class,
+                  b.act_rev, b.act_empty, b.attn_valid});
+}
+
+bool block_ok(const mantis_leaf_block& B) {
+  return all_set({B.u_w, B.mlp_w1_w, B.mlp_w2_w, B.mlp_w3_w, B.cr_kv_w, B.cr_q_w, B.cr_q_b, B.cr_o_w, B.cr_o_b,
+                  B.cr_bias, B.rad_kv_w, B.rad_q_w, B.rad_q_b, B.rad_o_w, B.rad_o_b, B.radius_bias, B.wr_kv_w,
+                  B.wr_q_w, B.wr_q_b, B.wr_o_w, B.wr_o_b, B.wr_bias, B.wproj_w, B.wproj_b, B.mlp_s1_w, B.mlp_s2_w,
+                  B.mlp_s3_w, B.qkv_w, B.attn_o_w, B.lq_read_x_w, B.lread_v_w, B.lread_v_b, B.lo_read_w, B.mix_qkv_wt,
+                  B.mix_qkv_b, B.mix_o_wt, B.mix_o_b, B.lkv_bcast_w, B.bcast_q_w, B.bcast_q_b, B.lo_bcast_w,
+                  B.lo_bcast_b, B.ffn1_w, B.ffn2_w}) &&
+         (B.cr_vcls == nullptr) == (B.rad_vcls == nullptr) &&
+         all_aligned({B.u_w, B.u_b, B.mlp_w1_w, B.mlp_w1_b, B.mlp_w2_w, B.ws_tab, B.mlp_w3_w, B.mlp_w3_b, B.cr_kv_w,
+                      B.cr_kv_b, B.cr_q_w, B.cr_q_b, B.cr_o_w, B.cr_o_b, B.cr_vcls, B.rad_kv_w, B.rad_kv_b, B.rad_q_w,
+                      B.rad_q_b, B.rad_o_w, B.rad_o_b, B.rad_vcls, B.wr_kv_w, B.wr_kv_b, B.wr_q_w, B.wr_q_b, B.wr_o_w,
+                      B.wr_o_b, B.wproj_w, B.wproj_b, B.mlp_s1_w, B.mlp_s1_b, B.mlp_s2_w, B.mlp_s3_w, B.mlp_s3_b,
+                      B.qkv_w, B.qkv_b, B.attn_o_w, B.attn_o_b, B.lq_read_x_w, B.lq_read_x_b, B.lread_v_w, B.lo_read_w,
+                      B.lo_read_b, B.lkv_bcast_w, B.lkv_bcast_b, B.bcast_q_w, B.bcast_q_b, B.lo_bcast_w, B.lo_bcast_b,
+                      B.ffn1_w, B.ffn1_b, B.ffn2_w, B.ffn2_b});
+}
+
+bool model_ok(const mantis_leaf_model& M, bool full) {
+  if (M.n_blocks < 1 || !M.blocks) return false;
+  for (int64_t i = 0; i < M.n_blocks; ++i)
+    if (!block_ok(M.blocks[i])) return false;
+  if (full && (M.n_bins < 1 || M.n_bins > 128 ||
+               !all_set({M.ln_value_w, M.ln_value_b, M.value_queries, M.mlp_v0_wt, M.mlp_v0_b, M.mlp_v2_wt, M.mlp_v2_b})))
+    return false;
+  for (int64_t n : {M.n_patterns, M.n_init, M.n_occ, M.n_dec_classes, M.n_rad_classes, M.n_act})
+    if (n < 1) return false;
+  return all_set({M.window_table, M.cell_table, M.stone_table, M.latent_base, M.token_moves, M.sw_all, M.ln_out_w,
+                  M.ln_out_b, M.act_proj_w, M.head1_w, M.head1_b, M.head2_w, M.head3_w, M.head3_b, M.act_table,
+                  M.empty_rows, M.head_tab, M.glin_wt}) &&
+         all_aligned({M.window_table, M.cell_table, M.stone_table, M.latent_base, M.token_moves, M.act_proj_w,
+                      M.act_proj_b, M.head1_w, M.head1_b, M.head2_w, M.head3_w, M.head3_b, M.act_table, M.empty_rows,
+                      M.head_tab});
+}
+
 }  // namespace
 }  // namespace mantis
 
@@ -419,10 +468,9 @@ int32_t mantis_leaf_forward(const mantis_leaf_model* model, const mantis_leaf_ba
   if (!model || !batch || !out || !workspace || !noncanonical || !tile_counters) return MANTIS_E_ARG;
   const mantis_leaf_model& M = *model;
   const mantis_leaf_batch& b = *batch;
-  if (!sizes_ok(b) || M.n_blocks < 1 || !M.blocks || !out->rows) return MANTIS_E_ARG;
   const bool full = out->value != nullptr;
-  if (full && (!out->policy || !out->q_values || !out->q_score || !out->dist || !out->logits || !out->bin_centers ||
-               M.n_bins < 1 || M.n_bins > 128))
+  if (!sizes_ok(b) || !batch_ok(b) || !model_ok(M, full) || !out->rows || !aligned16(out->rows)) return MANTIS_E_ARG;
+  if (full && !all_set({out->policy, out->q_values, out->q_score, out->dist, out->logits, out->bin_centers}))
     return MANTIS_E_ARG;
   const Space S(workspace, b, M.n_blocks);
   if (workspace_bytes < S.bytes || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return MANTIS_E_ARG;

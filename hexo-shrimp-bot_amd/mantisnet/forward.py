@@ -339,7 +339,8 @@ def _pack_leaf(cfg, t, P):
         x = x.detach()
         if x.dtype != HALF:
             x = x.float()
-        keep.append(x.contiguous())
+        x = x.contiguous()
+        keep.append(x.clone() if x.data_ptr() % 16 else x)  # (a parameter can be a view at any offset)
         return keep[-1].data_ptr()
 
     def block(pb):

@@ -108,3 +108,35 @@ def test_noalloc_size_guard_holds_at_int64_scale_counts():
                               (0, limit // 4 + 1)):
         rc = hip.mantis_stable_key_order_noalloc(fake, fake, fake, n_entries, n_keys, fake, fake, fake, None, None)
         assert rc == 3, (n_entries, n_keys, rc)
+
+
+def _leaf_call(**change):
+    """mantis_leaf_forward on stand-in addresses with one field changed."""
+    hip, a = _native.hip(), 0x10000
+    structs = {}
+    for name in ("Batch", "Block", "Model", "Out"):
+        struct = getattr(_hip_api, f"MantisLeaf{name}")
+        structs[name] = struct(**{f: a if t is _hip_api.vp else 8 for f, t in struct._fields_})
+    for k, v in change.items():
+        name, _, field = k.partition("_")
+        setattr(structs[name], field, v)
+    if structs["Model"].blocks:
+        structs["Model"].blocks = ctypes.addressof(structs["Block"])
+    structs["Model"].n_blocks = 1
+    by = ctypes.byref
+    return hip.mantis_leaf_forward(by(structs["Model"]), by(structs["Batch"]), by(structs["Out"]), 0.2, a, 1 << 40, a,
+                                   a, a, None)
+
+
+def test_leaf_forward_refuses_unset_fields_before_its_first_launch():
+    # the first kernel reads these without an entry point's check before it;
+    # without a device nothing can have been launched (2 would say it was tried)
+    cases = [{f"{n}_{f}": 0} for n in ("Batch", "Model", "Out") for f, t in
+             getattr(_hip_api, f"MantisLeaf{n}")._fields_
+             if t is _hip_api.vp and (n, f) not in (("Out", "value"), ("Model", "act_proj_b"))]
+    cases += [{f"Block_{f}": 0} for f, _ in _hip_api.MantisLeafBlock._fields_ if not f.endswith("_b") and f != "ws_tab"]
+    cases += [{f"Model_{f}": 0x10004} for f in ("stone_table", "latent_base", "token_moves", "window_table")]
+    cases += [{"Block_qkv_w": 0x10008}, {"Out_rows": 0x10008}, {"Batch_n_w": 0}, {"Model_n_init": 0}]
+    assert len(cases) > 90
+    for case in cases:
+        assert _leaf_call(**case) == 1, case
