@@ -4,48 +4,78 @@
 //   q|k|v = z Wqkv + bqkv                   (4 x 384)
 //   a_h  = softmax(q_h k_h^T / sqrt(32)) v_h  for each of the 4 heads of 32
 //   g_p += a Wo + bo
-// One workgroup of 1,024 threads per position.  The work is tiny (0.5 MFLOP
-// per position); what bounds it is fetching the weights (256 KB in fp32,
-// transposed so the threads read consecutive columns).  Every thread requests
-// all of its weights (80 values: a column's half of q|k|v, an eighth of an
-// output column) before its first row, so a launch waits for them once, and
-// keeps them across its positions.  With 256 threads reading 32 values at a
-// time it was five round trips one after the other: 13.8 us for one position
-// (now 7.9), 20 for 512 (17.9).
+// One workgroup of 512 threads per position, at most one per CU.  The work is
+// tiny (0.5 MFLOP per position); what bounds a launch is fetching the weights
+// (256 KB in fp32, transposed so the threads read consecutive columns) and the
+// chain of steps.  A thread requests all of its weights (one column of q|k|v
+// or of the output, 128 values) at once and keeps them across its positions.
+// Each projection is one fp32 FMA chain over k: the latents' last bits reach
+// every later 16-bit state, and sums cut into parts moved whole evaluations by
+// 9e-4.  The chains run on 4 x 4 x 1 fp32 MFMAs, half the issue time of vector
+// FMAs and a quarter of their LDS reads.  Per launch, weights in L2: 5.9 us for
+// one position, 11.6 for 512, 31 for 2,000 (chains of vector FMAs: 12.6, 27, 92;
+// 256 threads reading 32 weights at a time: 9.6, 13.4, 34; sums in 2 and 8
+// parts over 1,024 threads: 7.2, 16.8, 48).
 #include "common.hpp"
+#include "mfma.hpp"
 
 namespace mantis {
 namespace {
 
 constexpr int kH = 128;
 constexpr int kSlots = 4;
-constexpr int kThreads = 1024;
-constexpr int kParts = 8;  // cuts of the output projection's sums
+constexpr int kRowPitch = kH + 4;       // (the four rows' reads meet different banks)
+constexpr int kQkv = 3 * kH;            // threads [0, 384): a column of q|k|v each
+constexpr int kThreads = kQkv + kH;     // threads [384, 512): a column of the output each
+
+// The four rows' products with the wavefront's 64 weight columns (w: this
+// lane's), each one fp32 FMA chain over k in order: one 4 x 4 x 1 MFMA of 16
+// blocks per k (rows x this lane's quad of columns; lane 4 b + i brings row
+// i's value to block b, and holds its column's four sums).
+__device__ __forceinline__ f32x4_t column(const float (&x)[kSlots][kRowPitch], const float (&w)[kH], int lane) {
+  const float* mine = x[lane % 4];
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < kH; k += 4) {
+    const float4 v = *reinterpret_cast<const float4*>(mine + k);
+    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(v.x, w[k], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(v.y, w[k + 1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(v.z, w[k + 2], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(v.w, w[k + 3], acc, 0, 0, 0);
+  }
+  return acc;
+}
 
 __global__ void __launch_bounds__(kThreads)
 latent_mix_kernel(float* __restrict__ g, int64_t ldg, int64_t n_pos, const float* __restrict__ wqkv_t,
                   const float* __restrict__ bqkv, const float* __restrict__ wo_t, const float* __restrict__ bo,
                   float scale) {
-  __shared__ __attribute__((aligned(16))) float z[kSlots][kH];
-  __shared__ float part[kParts * kSlots * kH];  // q|k|v: [2][4][384], then the output: [8][4][128]
-  __shared__ float qkv[kSlots][3 * kH];
+  __shared__ __attribute__((aligned(16))) float z[kSlots][kRowPitch];
+  __shared__ float qkv[kSlots][kQkv];
   __shared__ float prob[4][kSlots][kSlots];  // [head][query][key]
-  __shared__ __attribute__((aligned(16))) float mixed[kSlots][kH];
-  static_assert(kParts * kSlots * kH >= 2 * kSlots * 3 * kH, "the partial products share one array");
+  __shared__ __attribute__((aligned(16))) float mixed[kSlots][kRowPitch];
   const int t = threadIdx.x, wave = t / 64, lane = t % 64;
-  // this thread's weights: column c1 of q|k|v over half the rows (the first
-  // 768 threads), column c2 of the output over an eighth
-  const int c1 = t % (3 * kH), half = t / (3 * kH), c2 = t % kH, oct = t / kH;
-  float w1[kH / 2], w2[kH / kParts];
+  // LayerNorm: wave w < 4 normalises row w, two features per lane.  A row is
+  // requested before the weights and, from then on, a position ahead (loads
+  // return in order: behind the weights it would wait for all of them)
+  float x0 = 0.f, x1 = 0.f;
+  auto request = [&](int64_t p) {
+    if (wave >= kSlots || p >= n_pos) return;
+    const float* row = g + (p * kSlots + wave) * ldg;
+    x0 = row[lane], x1 = row[lane + 64];
+  };
+  request(blockIdx.x);
+  // this thread's weight column (a wavefront is all of one kind)
+  const bool first = t < kQkv;
+  const int col = first ? t : t - kQkv, ldw = first ? kQkv : kH;
+  const float* from = (first ? wqkv_t : wo_t) + col;
+  float w[kH];
 #pragma unroll
-  for (int k = 0; k < kH / 2; ++k) w1[k] = half < 2 ? wqkv_t[(half * (kH / 2) + k) * 3 * kH + c1] : 0.f;
-#pragma unroll
-  for (int k = 0; k < kH / kParts; ++k) w2[k] = wo_t[(oct * (kH / kParts) + k) * kH + c2];
+  for (int k = 0; k < kH; ++k) w[k] = from[k * ldw];
+  const float b = first ? bqkv[col] : bo[col];
   for (int64_t p = blockIdx.x; p < n_pos; p += gridDim.x) {
     float* rows = g + p * kSlots * ldg;
-    // LayerNorm: wave w normalises row w, two features per lane
     if (wave < kSlots) {
-      const float x0 = rows[wave * ldg + lane], x1 = rows[wave * ldg + lane + 64];
       float s = x0 + x1;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
@@ -57,24 +87,14 @@ latent_mix_kernel(float* __restrict__ g, int64_t ldg, int64_t n_pos, const float
       const float rstd = rsqrtf(q * (1.f / kH) + 1e-5f);
       z[wave][lane] = d0 * rstd;
       z[wave][lane + 64] = d1 * rstd;
+      request(p + gridDim.x);
     }
     __syncthreads();
-    // q | k | v: column c1 of the four rows, over this thread's half of the sum
-    if (half < 2) {
-      float acc[kSlots] = {0.f, 0.f, 0.f, 0.f};
+    if (first) {
+      const f32x4_t acc = column(z, w, lane);
 #pragma unroll
-      for (int k = 0; k < kH / 2; k += 4)
-#pragma unroll
-        for (int r = 0; r < kSlots; ++r) {
-          const float4 x = *reinterpret_cast<const float4*>(&z[r][half * (kH / 2) + k]);
-          acc[r] = fmaf(x.w, w1[k + 3], fmaf(x.z, w1[k + 2], fmaf(x.y, w1[k + 1], fmaf(x.x, w1[k], acc[r]))));
-        }
-#pragma unroll
-      for (int r = 0; r < kSlots; ++r) part[(half * kSlots + r) * 3 * kH + c1] = acc[r];
+      for (int r = 0; r < kSlots; ++r) qkv[r][col] = acc[r] + b;
     }
-    __syncthreads();
-    for (int i = t; i < kSlots * 3 * kH; i += kThreads)
-      qkv[i / (3 * kH)][i % (3 * kH)] = part[i] + part[kSlots * 3 * kH + i] + bqkv[i % (3 * kH)];
     __syncthreads();
     // scores and softmax over the four keys: thread (head, query, key)
     if (t < 64) {
@@ -92,7 +112,7 @@ latent_mix_kernel(float* __restrict__ g, int64_t ldg, int64_t n_pos, const float
     }
     __syncthreads();
     // mixed[i][32 h + d] = sum_j prob[h][i][j] v[j][32 h + d]
-    if (t < kSlots * kH) {
+    {
       const int i = t / kH, c = t % kH, h = c / 32;
       float a = 0.f;
 #pragma unroll
@@ -100,28 +120,12 @@ latent_mix_kernel(float* __restrict__ g, int64_t ldg, int64_t n_pos, const float
       mixed[i][c] = a;
     }
     __syncthreads();
-    // output projection: column c2 of the four rows, over an eighth of the sum
-    {
-      float acc[kSlots] = {0.f, 0.f, 0.f, 0.f};
+    if (!first) {
+      const f32x4_t acc = column(mixed, w, lane);
 #pragma unroll
-      for (int k = 0; k < kH / kParts; k += 4)
-#pragma unroll
-        for (int r = 0; r < kSlots; ++r) {
-          const float4 x = *reinterpret_cast<const float4*>(&mixed[r][oct * (kH / kParts) + k]);
-          acc[r] = fmaf(x.w, w2[k + 3], fmaf(x.z, w2[k + 2], fmaf(x.y, w2[k + 1], fmaf(x.x, w2[k], acc[r]))));
-        }
-#pragma unroll
-      for (int r = 0; r < kSlots; ++r) part[(oct * kSlots + r) * kH + c2] = acc[r];
+      for (int r = 0; r < kSlots; ++r) rows[r * ldg + col] += acc[r] + b;
     }
-    __syncthreads();
-    if (t < kSlots * kH) {
-      const int r = t / kH;
-      float a = bo[c2];
-#pragma unroll
-      for (int k = 0; k < kParts; ++k) a += part[(k * kSlots + r) * kH + c2];
-      rows[r * ldg + c2] += a;
-    }
-    __syncthreads();  // z, part and qkv are rewritten by the next position
+    __syncthreads();  // z, qkv and the rows' next readers
   }
 }
 
@@ -138,7 +142,7 @@ extern "C" int32_t mantis_latent_mix(float* g, int64_t ldg, int64_t n_pos, const
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
                                               hipSuccess || cus <= 0)
     cus = 256;
-  const int64_t grid = n_pos < 4 * int64_t(cus) ? n_pos : 4 * int64_t(cus);
+  const int64_t grid = n_pos < cus ? n_pos : cus;  // one workgroup's weights fill a CU's registers
   latent_mix_kernel<<<dim3(unsigned(grid)), dim3(kThreads), 0, as_stream(stream)>>>(
       g, ldg, n_pos, wqkv_t, bqkv, wo_t, bo, 0.17677669529663687f);
   return launched();

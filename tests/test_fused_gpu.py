@@ -9,6 +9,8 @@ summation order plus one fp16 rounding of the output.
 
 from __future__ import annotations
 
+import ctypes
+import ctypes.util
 import math
 
 import pytest
@@ -988,6 +990,42 @@ def test_latent_mix_over_more_positions_than_workgroups(device):
     whole = ops.latent_mix(g.clone(), w, b, wo, bo)
     assert torch.equal(ops.latent_mix(g[:4].clone(), w, b, wo, bo), whole[:4])
     assert torch.equal(ops.latent_mix(g[4096:].clone(), w, b, wo, bo), whole[4096:])
+
+
+def test_latent_mix_sums_every_product_in_one_chain(device):
+    # the projections are one fp32 FMA chain over k each, in order: a state of
+    # several 16-bit layers follows the last bits of these sums.  Weights of
+    # 2^60 hide the residual row; latents of zeros leave the first one's value
+    # at a quarter, and without any other latent the biases as they are.
+    fmaf = ctypes.CDLL(ctypes.util.find_library("m")).fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+
+    def chain(x, w):  # (128,), (128, n)
+        out = []
+        for c in range(w.shape[1]):
+            acc = 0.0
+            for a, b in zip(x.tolist(), w[:, c].tolist()):
+                acc = fmaf(a, b, acc)
+            out.append(acc)
+        return torch.tensor(out)
+
+    gen = _g(20)
+    big, eye = 2.0 ** 60, torch.eye(128)
+
+    def mix(g, wv, bv, wo, bo):
+        w = torch.cat([torch.zeros(128, 256), wv], 1)
+        b = torch.cat([torch.zeros(256), bv])
+        return ops.latent_mix(*(t.to(device).contiguous() for t in (g, w, b, wo, bo))).cpu()
+
+    g = torch.zeros(4, 128)
+    g[0] = torch.where(torch.randperm(128, generator=gen) < 64, 1.0, -1.0)
+    zero = torch.zeros(128)
+    z = mix(g, big * eye, zero, eye, zero)[1] * (4 / big)
+    wv = torch.randn(128, 128, generator=gen)
+    assert torch.equal(mix(g, big * wv, zero, eye, zero)[1] * (4 / big), chain(z, wv))
+    bv = torch.randint(-63, 64, (128,), generator=gen) / 16
+    wo, bo = torch.randn(128, 128, generator=gen), torch.randn(128, generator=gen)
+    assert torch.equal(mix(torch.zeros(4, 128), wv, bv, wo, bo)[2], chain(bv, wo) + bo)
 
 
 def test_latent_mix_matches_the_fp32_formulation(device):
