@@ -444,7 +444,7 @@ def window_latent_read_backward(q: Tensor, k: Tensor, v: Tensor, window_pos: Ten
                                 out: Tensor, m: Tensor, l: Tensor,
                                 grad_out: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     """(dq, dk, dv) of window_latent_read."""
-    return ops.latent_read_backward(q, k, v, window_pos, offsets, order, out, m, l, grad_out)
+    return ops.latent_read_backward(q, k, v, window_pos, offsets, order, m, l, grad_out, out)
 
 
 @window_latent_read_backward.register_fake

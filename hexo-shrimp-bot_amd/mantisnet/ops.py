@@ -715,9 +715,12 @@ def _latent_backward(q, k, v, n_q, n_k, window_pos, offsets, order, m, l, grad_o
     return dq.view(q.shape), dk.view(k.shape), dv.view(v.shape)
 
 
-def latent_read_backward(q, k, v, window_pos, offsets, order, out, m, l, grad_out):
+def latent_read_backward(q, k, v, window_pos, offsets, order, m, l, grad_out, out=None):
     """(dq, dk, dv) of latent_read: the four slot queries of each position
-    over its windows (window_latents.py:132-163); out, m and l the forward's."""
+    over its windows (window_latents.py:132-163); m, l and out the forward's
+    (without out it is formed again)."""
+    if out is None:
+        out = latent_read(q, k, v, offsets, order)
     return _latent_backward(q, k, v, q.shape[0] * 4, k.shape[0], window_pos, offsets, order, m, l, grad_out, out)
 
 

@@ -196,6 +196,19 @@ def test_window_latent_backward_takes_any_order(device):
     mantisnet.ops.raise_on_device_error(device)
 
 
+def test_latent_read_backward_without_the_forward_output(device):
+    # the module-level call as it was: m, l and the gradient, out formed again
+    gen = torch.Generator().manual_seed(28)
+    window_pos = torch.tensor([0] * 70 + [2] * 9)
+    offsets, order = R.window_layout(window_pos, 3)
+    q, k, v, go = (torch.randn(*s, generator=gen).to(device) for s in ((3, 4, 4, 32), (79, 4, 32), (79, 4, 32),
+                                                                     (3, 4, 4, 32)))
+    layout = [x.to(device) for x in (window_pos, offsets, order)]
+    out, m, l = OPS.window_latent_read(q, k, v, *layout)
+    got = mantisnet.ops.latent_read_backward(q, k, v, *layout, m, l, go)
+    assert all(torch.equal(a, b) for a, b in zip(got, OPS.window_latent_read_backward(q, k, v, *layout, out, m, l, go)))
+
+
 def test_action_row_encode_backward(device, batch):
     b = batch
     n_w, n_c = b.window_feat.numel(), b.cell_pos.shape[0]
