@@ -874,8 +874,9 @@ int32_t mantis_run_reduce(const void* values, int32_t values_dtype, int64_t n_sr
                                                         n_dest, n_entries, static_cast<TO*>(out), err_flag);
       else if (vec) {
         // (the reason for either number of rows in flight is at the kernel)
-        const auto kernel = sizeof(TI) == 2 && n_entries >= 4 * n_dest ? run_reduce_kernel<TI, TO, 8>
-                                                                       : run_reduce_kernel<TI, TO, 4>;
+        auto kernel = run_reduce_kernel<TI, TO, 4>;
+        if constexpr (sizeof(TI) == 2)
+          if (n_entries >= 4 * n_dest) kernel = run_reduce_kernel<TI, TO, 8>;
         const dim3 chunks(grid.x, unsigned(std::min<int64_t>((h + 127) / 128, 65535)));
         kernel<<<chunks, block, 0, s>>>(static_cast<const TI*>(values), n_src, ld, h, gather, ptr, n_dest, n_entries,
                                         static_cast<TO*>(out), err_flag);

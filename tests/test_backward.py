@@ -138,6 +138,34 @@ def test_cell_attention_backward_run_lengths(device, n_k, dt, with_vcls):
     assert all(torch.equal(a, b) for a, b in zip(got, again))
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_attention_backward_without_classes_or_query_ids(device, dt):
+    """The module-level forms that the operators do not take: untyped entries
+    are entries of one class without a bias, and without the entries' query
+    ids the query pass itself finishes the bias gradient's terms."""
+    gen = torch.Generator().manual_seed(29)
+    n_q, n_k, n_e = 21, 13, 160
+    dst, src = torch.randint(3, n_q, (n_e,), generator=gen), torch.randint(0, n_k, (n_e,), generator=gen)
+    q, k, v = (torch.randn(n, 4, 32, generator=gen).to(device, dt) for n in (n_q, n_k, n_k))
+    go = torch.randn(n_q, 4, 32, generator=gen).to(device)
+    back = mantisnet.ops.attention_backward
+    for n_cls in (1, 3):
+        t = R.edge_tables_full(src, dst, torch.randint(0, n_cls, (n_e,), generator=gen), dst[:0], n_k, n_q, n_cls, False)
+        bias = torch.zeros(4, n_cls, device=device)
+        views = [t[n].to(device) for n in ("dst_ptr", "edge_src", "edge_class", "edge_dst", "source_ptr", "edge_sdst",
+                                           "edge_sclass", "cls_ptr", "cedge_dst")]
+        _, m, l = OPS.cell_attention_plain(q, k, v, bias, *views)
+        full = OPS.cell_attention_plain_backward(q, k, v, bias, *views, m, l, go)
+        seg, es, ec, _, sseg, sqid, scls, cptr, cedge = views
+        no_qid = back(q, k, v, bias, None, go, m, l, seg, es, ec, None, sseg, sqid, scls, cptr, cedge)
+        assert all(torch.equal(a, b) for a, b in zip(no_qid[:3], full))
+        # fp32 sums of 160 terms of up to about 5 each
+        torch.testing.assert_close(no_qid[3], full[3], rtol=0, atol=5e-5)
+        untyped = back(q, k, v, None, None, go, m, l, seg, es, None, None, sseg, sqid, None, None, None)
+        assert all(torch.equal(a, b) for a, b in zip(untyped[:3], full)) and untyped[3] is None and untyped[4] is None
+    mantisnet.ops.raise_on_device_error(device)
+
+
 @pytest.mark.parametrize("counts,dt,shuffled", [
     ([0], torch.float32, False), ([1], torch.float32, False), ([63, 64, 65], torch.float32, True),
     ([3, 0, 700, 17], torch.float32, True), ([130, 1, 0], torch.bfloat16, False), ([16, 15, 257], torch.float16, True),
