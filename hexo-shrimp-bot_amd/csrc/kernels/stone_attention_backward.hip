@@ -10,21 +10,24 @@
 // and transposed, the next chunk's in registers meanwhile:
 //   query-major  S^T = K Q^T and dP^T = V dO^T, then dQ^T += K^T dS^T
 //   key-major    S = Q K^T and dP = dO V^T, then dV^T += dO^T P, dK^T += Q^T dS
-// Both keep a lane on one row of its own side, so a score fragment is the next
-// product's B operand (K slots {4g..4g+3, 16+4g..16+4g+3}, the transposed rows
-// read in the same order).
+// Both keep a lane on one row of its own side, so a score fragment's value of
+// row 16 tt + 4 g + t is the next product's B operand as it stands (the four
+// K slots of a step are the rows 4 g + t of the lane groups g).
 //
-// Precision: scores and dp are exact products of 16-bit rows summed in fp32.
-// The probabilities and ds stay fp32 values: each enters its product as a
-// bf16 pair hi + lo (16 significant bits, the full exponent range), two MFMAs
-// instead of one.  fp16 rows enter those products as bf16 pairs too (exact),
-// a third MFMA; fp16 pairs of ds would lose small gradients to underflow.
-// Every sum is fp32 in a fixed order: two calls agree bitwise.  Rows and keys
-// at or past L get zero gradients.
+// Precision: scores and dp are exact products of 16-bit rows summed in fp32
+// (16-bit MFMA); the probabilities and ds are fp32 and enter their products,
+// with the rows widened, as fp32 MFMA operands.  Every sum is fp32 in a fixed
+// order: two calls agree bitwise.  Rows and keys at or past L get zero
+// gradients, whatever the live rows hold.
 //
-// Bound by the VALU work per score (one exp2, the pair splits) and the chunk
-// latency; 192 positions of 44-124 rows, 4 heads of 32, bf16: one row per lane
-// with fp32 FMAs took 77 and 150 us, these passes take 15 and 17.
+// Bound by the latency of a wavefront's own chain per chunk (rows, barrier,
+// products, exponentials, then 32 or 64 dependent fp32 MFMAs) with two
+// wavefronts per SIMD: MFMA 12-18% busy, VALU 17-18%, half of the wavefronts'
+// time waiting.  192 positions of 44-124 rows, 4 heads of 32, bf16: one row per
+// lane with fp32 FMAs took 74 and 152 us, these passes take 20 and 28; 16
+// positions of 512-1,024 rows 390 and 611, now 64 and 105.  (Operands cut to
+// bf16 pairs of 16 significant bits: 15 and 17, 40 and 55, but sums that cancel
+// lose those bits and an infinite row turned zeros into NaNs.)
 #include "common.hpp"
 #include "mfma.hpp"
 
@@ -52,15 +55,6 @@ __device__ __forceinline__ float widen(uint32_t bits) {
   else return __uint_as_float(bits << 16);
 }
 
-// x as a bf16 pair, two values at a time: hi truncated, so lo has x's sign (a
-// non-finite row then leaves non-finite sums in its own dims only); hi + lo
-// holds 16 significant bits
-__device__ __forceinline__ void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
-  const uint32_t bx = __float_as_uint(x) & 0xffff0000u, by = __float_as_uint(y) & 0xffff0000u;
-  hi = (bx >> 16) | by;
-  lo = pack_bf16x2(x - __uint_as_float(bx), y - __uint_as_float(by));
-}
-
 template <bool kHalf, int HD>
 struct Geom {
   static constexpr int kPitch = HD + 8;                 // 16-bit elements per staged row
@@ -68,14 +62,12 @@ struct Geom {
   static constexpr int kDt = HD / 16;                   // 16-dim output tiles
   static constexpr int kPieces = kTile * HD / 8;        // 16-byte pieces of a chunk
   static constexpr int kPer = kPieces < 256 ? 1 : kPieces / 256;
-  static constexpr int kTerms = kHalf ? 2 : 1;          // bf16 terms of a transposed row
-  // the dims of this lane in K step ks (HD = 16: lanes g >= 2 repeat the dims
-  // of g - 2 and hold zeros in the B operand)
+  // the dims of this lane in K step ks (HD = 16: lanes g >= 2 hold zeros)
   static __device__ __forceinline__ int kdim(int ks, int g) { return HD < 32 ? 8 * (g & 1) : 32 * ks + 8 * g; }
 };
 
 // A 64-row chunk of one operand: fetched to registers (zeros at or past L),
-// staged as rows, as transposed rows of bf16 terms, or both.
+// staged as rows, as transposed rows, or both.
 template <bool kHalf, int HD>
 struct Chunk {
   using G = Geom<kHalf, HD>;
@@ -106,14 +98,8 @@ struct Chunk {
       const uint32_t w[4] = {reg[r].x, reg[r].y, reg[r].z, reg[r].w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        uint32_t hi = w[e], lo = 0;
-        if constexpr (kHalf) split2(widen<true>(w[e] & 0xffffu), widen<true>(w[e] >> 16), hi, lo);
-        col[2 * e * kTPitch] = uint16_t(hi);
-        col[(2 * e + 1) * kTPitch] = uint16_t(hi >> 16);
-        if constexpr (kHalf) {
-          col[(HD + 2 * e) * kTPitch] = uint16_t(lo);
-          col[(HD + 2 * e + 1) * kTPitch] = uint16_t(lo >> 16);
-        }
+        col[2 * e * kTPitch] = uint16_t(w[e]);
+        col[(2 * e + 1) * kTPitch] = uint16_t(w[e] >> 16);
       }
     }
   }
@@ -131,53 +117,47 @@ __device__ __forceinline__ void load_frags(const uint16_t* row, bool live, int g
   }
 }
 
-// 4 tiles of 16 staged rows times this lane's row
+// 4 tiles of 16 staged rows times this lane's row, those with a row below n (HD = 16: the upper K slots
+// are zeros on both sides, so an infinite row meets none of them)
 template <bool kHalf, int HD>
-__device__ __forceinline__ void products(const uint16_t* s, int l16, int g, const uint4 (&b)[Geom<kHalf, HD>::kKs],
+__device__ __forceinline__ void products(const uint16_t* s, int n, int l16, int g, const uint4 (&b)[Geom<kHalf, HD>::kKs],
                                          f32x4_t (&d)[4]) {
   using G = Geom<kHalf, HD>;
   using FR = Frag<kHalf>;
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt) {
     d[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (16 * tt >= n) continue;  // uniform
 #pragma unroll
     for (int ks = 0; ks < G::kKs; ++ks) {
-      const uint4 a = *reinterpret_cast<const uint4*>(s + (16 * tt + l16) * G::kPitch + G::kdim(ks, g));
+      uint4 a = *reinterpret_cast<const uint4*>(s + (16 * tt + l16) * G::kPitch + G::kdim(ks, g));
+      if (HD < 32 && g >= 2) a = make_uint4(0u, 0u, 0u, 0u);
       d[tt] = mfma16x16x32(FR::cast(a), FR::cast(b[ks]), d[tt]);
     }
   }
 }
 
-// acc (HD dims x this lane's row) += transposed rows . x over a chunk's 64 rows,
-// x the 16 fp32 values of this lane (rows 16 tt + 4 g + t)
+// acc (HD dims x this lane's row) += transposed rows . x over a chunk's tiles with
+// a row below n, x the 16 fp32 values of this lane (rows 16 tt + 4 g + t), on the fp32 MFMA
+// (16 x 16 x 4: lane group g holds K slot g of both operands)
 template <bool kHalf, int HD>
-__device__ __forceinline__ void accumulate(const uint16_t* st, int l16, int g, const float (&x)[4][4],
+__device__ __forceinline__ void accumulate(const uint16_t* st, int n, int l16, int g, const float (&x)[4][4],
                                            f32x4_t (&acc)[Geom<kHalf, HD>::kDt]) {
-  using G = Geom<kHalf, HD>;
 #pragma unroll
-  for (int sc = 0; sc < 2; ++sc) {
-    uint32_t hi[4], lo[4];
+  for (int tt = 0; tt < 4; ++tt) {
+    if (16 * tt >= n) break;  // uniform
+    uint2 a[Geom<kHalf, HD>::kDt];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int tt = 2 * sc + e / 2, t = 2 * (e % 2);
-      split2(x[tt][t], x[tt][t + 1], hi[e], lo[e]);
-    }
-    const bf16x8_t bh = as_bf16x8(make_uint4(hi[0], hi[1], hi[2], hi[3]));
-    const bf16x8_t bl = as_bf16x8(make_uint4(lo[0], lo[1], lo[2], lo[3]));
+    for (int dt = 0; dt < Geom<kHalf, HD>::kDt; ++dt)
+      a[dt] = *reinterpret_cast<const uint2*>(st + (16 * dt + l16) * kTPitch + 16 * tt + 4 * g);
 #pragma unroll
-    for (int dt = 0; dt < G::kDt; ++dt) {
-      const uint16_t* row = st + (16 * dt + l16) * kTPitch + 32 * sc;
-      const uint2 p0 = *reinterpret_cast<const uint2*>(row + 4 * g);
-      const uint2 p1 = *reinterpret_cast<const uint2*>(row + 16 + 4 * g);
-      const bf16x8_t a = as_bf16x8(make_uint4(p0.x, p0.y, p1.x, p1.y));
-      acc[dt] = mfma16x16x32(a, bl, acc[dt]);
-      if constexpr (kHalf) {
-        const uint2 q0 = *reinterpret_cast<const uint2*>(row + HD * kTPitch + 4 * g);
-        const uint2 q1 = *reinterpret_cast<const uint2*>(row + HD * kTPitch + 16 + 4 * g);
-        acc[dt] = mfma16x16x32(as_bf16x8(make_uint4(q0.x, q0.y, q1.x, q1.y)), bh, acc[dt]);
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int dt = 0; dt < Geom<kHalf, HD>::kDt; ++dt) {
+        const uint32_t w = t < 2 ? a[dt].x : a[dt].y;
+        const float v = widen<kHalf>(t % 2 ? w >> 16 : w & 0xffffu);
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, x[tt][t], acc[dt], 0, 0, 0);
       }
-      acc[dt] = mfma16x16x32(a, bh, acc[dt]);
-    }
   }
 }
 
@@ -202,7 +182,7 @@ stone_bwd_q_kernel(Rows q, Rows k, Rows v, Rows o, Rows go, const int32_t* __res
                    int64_t T, const float* __restrict__ lse, float scale, float* __restrict__ delta, RowsOut dq) {
   using G = Geom<kHalf, HD>;
   __shared__ __attribute__((aligned(16))) uint16_t sk[kTile * G::kPitch], sv[kTile * G::kPitch];
-  __shared__ __attribute__((aligned(16))) uint16_t skt[G::kTerms * HD * kTPitch];
+  __shared__ __attribute__((aligned(16))) uint16_t skt[HD * kTPitch];
   const int64_t n_tiles = (T + kTile - 1) / kTile;
   const int64_t pa = blockIdx.x / n_tiles, tile = blockIdx.x % n_tiles;
   const int64_t pos = pa / heads, a = pa % heads;
@@ -215,7 +195,7 @@ stone_bwd_q_kernel(Rows q, Rows k, Rows v, Rows o, Rows go, const int32_t* __res
   load_frags<kHalf, HD>(q.at(pos, a) + i * q.st, live, g, qf);
   load_frags<kHalf, HD>(go.at(pos, a) + i * go.st, live, g, gf);
   load_frags<kHalf, HD>(o.at(pos, a) + i * o.st, live, g, of);
-  const float lse2 = live ? lse[pa * T + i] * kLog2e : 0.f;
+  const float li = live ? lse[pa * T + i] : 0.f;
   float dl = 0.f;
 #pragma unroll
   for (int ks = 0; ks < G::kKs; ++ks) {
@@ -233,7 +213,6 @@ stone_bwd_q_kernel(Rows q, Rows k, Rows v, Rows o, Rows go, const int32_t* __res
   if (tile * kTile < L) {  // workgroup-uniform: some row of the tile is live
     const uint16_t* kp = k.at(pos, a);
     const uint16_t* vp = v.at(pos, a);
-    const float c_log2 = scale * kLog2e;
     Chunk<kHalf, HD> ck, cv;
     ck.fetch(kp, k.st, 0, L);
     cv.fetch(vp, v.st, 0, L);
@@ -249,18 +228,19 @@ stone_bwd_q_kernel(Rows q, Rows k, Rows v, Rows o, Rows go, const int32_t* __res
       }
       if (first >= L) continue;  // wavefront-uniform: no live row here
       f32x4_t s[4], dp[4];
-      products<kHalf, HD>(sk, l16, g, qf, s);
-      products<kHalf, HD>(sv, l16, g, gf, dp);
-      const int lim = int(L - kb) - 4 * g;  // keys 16 tt + t below it are live
+      const int n = int(L - kb < kTile ? L - kb : kTile);
+      products<kHalf, HD>(sk, n, l16, g, qf, s);
+      products<kHalf, HD>(sv, n, l16, g, gf, dp);
+      const int lim = n - 4 * g;  // keys 16 tt + t below it are live
       float ds[4][4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const float al = __builtin_amdgcn_exp2f(fmaf(s[tt][t], c_log2, -lse2));
+          const float al = __builtin_amdgcn_exp2f(fmaf(s[tt][t], scale, -li) * kLog2e);
           ds[tt][t] = 16 * tt + t < lim ? al * (dp[tt][t] - dl) : 0.f;
         }
-      accumulate<kHalf, HD>(skt, l16, g, ds, acc);
+      accumulate<kHalf, HD>(skt, n, l16, g, ds, acc);
     }
   }
   if (i < T) {
@@ -276,7 +256,7 @@ stone_bwd_kv_kernel(Rows q, Rows k, Rows v, Rows go, const int32_t* __restrict__
                     RowsOut dv) {
   using G = Geom<kHalf, HD>;
   __shared__ __attribute__((aligned(16))) uint16_t sq[kTile * G::kPitch], sg[kTile * G::kPitch];
-  __shared__ __attribute__((aligned(16))) uint16_t sqt[G::kTerms * HD * kTPitch], sgt[G::kTerms * HD * kTPitch];
+  __shared__ __attribute__((aligned(16))) uint16_t sqt[HD * kTPitch], sgt[HD * kTPitch];
   __shared__ __attribute__((aligned(16))) float sl[kTile], sd[kTile];
   const int64_t n_tiles = (T + kTile - 1) / kTile;
   const int64_t pa = blockIdx.x / n_tiles, tile = blockIdx.x % n_tiles;
@@ -295,16 +275,14 @@ stone_bwd_kv_kernel(Rows q, Rows k, Rows v, Rows go, const int32_t* __restrict__
   if (tile * kTile < L) {  // workgroup-uniform
     const uint16_t* qp = q.at(pos, a);
     const uint16_t* gp = go.at(pos, a);
-    const float c_log2 = scale * kLog2e;
     Chunk<kHalf, HD> cq, cg;
     float rl = 0.f, rd = 0.f;
     auto fetch = [&](int64_t qb) {
       cq.fetch(qp, q.st, qb, L);
       cg.fetch(gp, go.st, qb, L);
       if (threadIdx.x < kTile) {
-        // a dead row's probabilities are exp2(0 - inf) = 0
         const bool in = qb + threadIdx.x < L;
-        rl = in ? lse[pa * T + qb + threadIdx.x] * kLog2e : INFINITY;
+        rl = in ? lse[pa * T + qb + threadIdx.x] : 0.f;
         rd = in ? delta[pa * T + qb + threadIdx.x] : 0.f;
       }
     };
@@ -323,8 +301,10 @@ stone_bwd_kv_kernel(Rows q, Rows k, Rows v, Rows go, const int32_t* __restrict__
       if (qb + kTile < L) fetch(qb + kTile);
       if (first >= L) continue;  // wavefront-uniform
       f32x4_t s[4], dp[4];
-      products<kHalf, HD>(sq, l16, g, kf, s);
-      products<kHalf, HD>(sg, l16, g, vf, dp);
+      const int n = int(L - qb < kTile ? L - qb : kTile);
+      products<kHalf, HD>(sq, n, l16, g, kf, s);
+      products<kHalf, HD>(sg, n, l16, g, vf, dp);
+      const int lim = n - 4 * g;  // queries 16 tt + t below it are live
       float al[4][4], ds[4][4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
@@ -333,12 +313,13 @@ stone_bwd_kv_kernel(Rows q, Rows k, Rows v, Rows go, const int32_t* __restrict__
         const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dv4[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          al[tt][t] = __builtin_amdgcn_exp2f(fmaf(s[tt][t], c_log2, -lv[t]));
-          ds[tt][t] = al[tt][t] * (dp[tt][t] - dv4[t]);
+          const float e = __builtin_amdgcn_exp2f(fmaf(s[tt][t], scale, -lv[t]) * kLog2e);
+          al[tt][t] = 16 * tt + t < lim ? e : 0.f;
+          ds[tt][t] = 16 * tt + t < lim ? e * (dp[tt][t] - dv4[t]) : 0.f;
         }
       }
-      accumulate<kHalf, HD>(sgt, l16, g, al, av);
-      accumulate<kHalf, HD>(sqt, l16, g, ds, ak);
+      accumulate<kHalf, HD>(sgt, n, l16, g, al, av);
+      accumulate<kHalf, HD>(sqt, n, l16, g, ds, ak);
     }
   }
   if (j < T) {

@@ -313,3 +313,75 @@ def test_fused_attention_backward_tiles(device, hd, dt, grad_scale):
         g, e = g.cpu().double(), e.masked_fill(~valid, 0.0)
         assert float((g - e).norm() / e.norm()) < 2 * tol + 1e-7 / grad_scale
         assert torch.count_nonzero(g.masked_fill(valid, 0.0)) == 0
+
+
+def _attention_backward_terms(q, k, v, lens, lse, go, out, scale):
+    """P, dS (heads, L, L) and the live rows of each position in float64."""
+    for p, n in enumerate(lens.tolist()):
+        a, b, c, g, o = (x[p, :, :n].double() for x in (q, k, v, go, out))
+        pr = torch.exp(a @ b.transpose(1, 2) * scale - lse[p, :, :n].double()[..., None])
+        yield p, n, a, b, g, pr, pr * (g @ c.transpose(1, 2) - (o * g).sum(-1)[..., None])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd", [16, 32, 64])
+def test_fused_attention_backward_keeps_fp32_probabilities(device, hd, dt):
+    """Queries in pairs a few 16-bit steps apart with opposite gradients: dv and
+    dk are 2^-7 and less of their terms, so what a product loses of P or dS
+    shows through the output's rounding.  Past half a rounding step the error
+    stays within 2^-20 of the terms' root sum of squares: fp32 operands leave
+    2^-22 of the exponent's argument and 2^-25 of the sums, operands of 16
+    significant bits leave 2^-17."""
+    gen = torch.Generator().manual_seed(50 + hd)
+    lens = torch.tensor([2, 8, 64, 66, 128], dtype=torch.int32)
+    p, t, heads, scale = len(lens), 130, 2, hd ** -0.5
+    q, go = (torch.randn(p, heads, t // 2, hd, generator=gen).repeat_interleave(2, 2) for _ in range(2))
+    q[:, :, 1::2] += 2 ** -9 * torch.randn(p, heads, t // 2, hd, generator=gen)
+    go[:, :, 1::2] *= -1
+    k, v = (torch.randn(p, heads, t, hd, generator=gen) for _ in range(2))
+    q, k, v, go = (x.to(dt) for x in (q, k, v, go))
+    out, lse = torch.zeros_like(q), torch.zeros(p, heads, t)
+    for i, n in enumerate(lens.tolist()):
+        s = q[i, :, :n].double() @ k[i, :, :n].double().transpose(1, 2) * scale
+        lse[i, :, :n] = s.logsumexp(-1).float()
+        out[i, :, :n] = (s.softmax(-1) @ v[i, :, :n].double()).to(dt)
+    dq, dk, dv = (x.cpu().double() for x in OPS.fused_attention_backward(
+        *(x.to(device) for x in (q, k, v, lens, out, lse, go))))
+    half = 2 ** -8 if dt == torch.bfloat16 else 2 ** -11
+    worst = {}
+    for i, n, a, b, g, pr, ds in _attention_backward_terms(q, k, v, lens, lse, go, out, scale):
+        for name, got, x, rows, f in (("dv", dv, pr.transpose(1, 2), g, 1.0),
+                                      ("dk", dk, ds.transpose(1, 2), a, scale), ("dq", dq, ds, b, scale)):
+            exp = x @ rows * f
+            terms = f * ((x ** 2) @ (rows ** 2)).sqrt()
+            over = ((got[i, :, :n] - exp).abs() - half * exp.abs() - 2 ** -25).clamp(min=0)  # (fp16 below 2^-14)
+            worst[name, n] = float((over ** 2).mean().sqrt() / (terms ** 2).mean().sqrt())
+    print(hd, dt, {k: f"{v:.1e}" for k, v in worst.items()}, flush=True)
+    assert max(worst.values()) < 2 ** -20, worst
+
+
+@pytest.mark.parametrize("hd", [16, 32, 64])
+def test_fused_attention_backward_of_a_masked_key(device, hd):
+    """A key of -inf scores (P = 0 on every row) gets zero gradients, and the
+    rows past the prefix bring none to it; an infinite P leaves infinities of
+    the gradient's sign."""
+    gen = torch.Generator().manual_seed(60 + hd)
+    n, t, scale = 3, 70, hd ** -0.5
+    lens = torch.tensor([n], dtype=torch.int32)
+    q, k, v, go = (torch.randn(1, 1, t, hd, generator=gen).bfloat16() for _ in range(4))
+    q[..., 0] = q[..., 0].abs() + 1
+    k[0, 0, 1, 0] = float("-inf")
+    s = q[0, 0, :n].double() @ k[0, 0, :n].double().t() * scale
+    lse, out = torch.zeros(1, 1, t), torch.zeros_like(q)
+    lse[0, 0, :n] = s.logsumexp(-1).float()
+    out[0, 0, :n] = (s.softmax(-1) @ v[0, 0, :n].double()).bfloat16()
+    args = [x.to(device) for x in (q, k, v, lens, out, lse, go)]
+    dq, dk, dv = (x.cpu().double() for x in OPS.fused_attention_backward(*args))
+    assert not dk[0, 0, 1].any() and not dv[0, 0, 1].any()
+    for i, m, a, b, g, pr, ds in _attention_backward_terms(q, k, v, lens, lse, go, out, scale):
+        torch.testing.assert_close(dv[i, :, :m], pr.transpose(1, 2) @ g, rtol=2 ** -8, atol=1e-6)
+        torch.testing.assert_close(dk[i, :, :m], ds.transpose(1, 2) @ a * scale, rtol=2 ** -8, atol=1e-6)
+        torch.testing.assert_close(dq[i, :, :m, 1:], (ds @ b * scale)[..., 1:], rtol=2 ** -8, atol=1e-6)
+    args[3], args[5] = torch.ones_like(args[3]), torch.full_like(args[5], -500.0)
+    dv = OPS.fused_attention_backward(*args)[2].cpu().float()
+    assert torch.equal(dv[0, 0, 0], torch.copysign(torch.tensor(float("inf")), go[0, 0, 0].float()))
