@@ -281,6 +281,27 @@ def test_class_reduce_run_lengths(device, h, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_classes", [1023, 1024, 1031])
+@pytest.mark.parametrize("h,odt", [(8, torch.float32), (20, torch.float32), (128, torch.bfloat16), (264, torch.float32)])
+def test_class_reduce_of_many_classes(device, n_classes, h, odt):
+    """Either side of the merge's 1,024 runs and of its 8 runs per workgroup:
+    runs of no entry, of one, around 8 partial rows (512 entries) and one that
+    owns most entries, the longer ones in one workgroup and apart."""
+    gen = torch.Generator().manual_seed(15)
+    lens = torch.randint(0, 4, (n_classes,), generator=gen)
+    lens[[3, 4, 5, 6, 700, -1]] = torch.tensor([512, 513, 577, 64, 9000, 1100])
+    cls_ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    values = torch.randn(300, h, generator=gen)
+    rows = torch.randint(0, 300, (int(lens.sum()),), generator=gen)
+    cls = torch.repeat_interleave(torch.arange(n_classes), lens)
+    got = mantisnet.ops.class_reduce(values.to(device), rows.to(device), cls_ptr.to(device), n_classes, odt)
+    mantisnet.ops.raise_on_device_error(device)
+    ref = torch.zeros(n_classes, h, dtype=torch.float64).index_add_(0, cls, values.double()[rows])
+    # fp32 sums of n values near 1, rounded once to odt
+    torch.testing.assert_close(got.double().cpu(), ref, rtol=1e-5 if odt == torch.float32 else 2 ** -8, atol=1e-3)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,n_keys", [(0, 5), (1, 1), (63, 2), (512, 726), (513, 729), (4097, 1458),
                                       (70001, 2048), (3000, 2049)])
 def test_class_order(device, n, n_keys):
