@@ -1,11 +1,11 @@
 // Sliced reductions over unbounded runs (class-major entry lists, where one
 // class can own most of the entries): every run is cut into slices of at
 // most kSlice entries, each slice is summed into a partial row by its own
-// lane group, and slice_merge_kernel sums each run's partials, a workgroup
-// per run and 32 columns.  The slice tables come from two small kernels: an
-// exclusive scan of the slice counts (slice_ptr, one per run) and the first
-// entry of every slice (slice_edge).  Deterministic: fixed slice bounds,
-// fixed orders.
+// lane group, and slice_merge sums each run's partials, a workgroup per run
+// and 32 columns or, of many short runs, per 8 runs.  The slice tables come
+// from two small kernels: an exclusive scan of the slice counts (slice_ptr,
+// one per run) and the first entry of every slice (slice_edge).
+// Deterministic: fixed slice bounds, fixed orders.
 #pragma once
 
 #include "common.hpp"
@@ -229,15 +229,18 @@ slice_merge_many_kernel(const float* __restrict__ partial, int64_t h, const int6
   }
 }
 
-// A workgroup per run and 32 columns while runs are few or long; from 1,024 runs
-// of at most 8 partial rows on average, 8 runs each: class sums of 100,000
-// entries over 20,000 classes take 57 us instead of 95, of 200,000 over 100,000
-// classes 214 instead of 405, of 100,000 over 2,000 25 instead of 29 (a lane group
-// per run, as before the merge: 63, 217 and 67).
+// A workgroup per run and 32 columns for up to 2,048 runs (the class
+// vocabularies, a few of whose classes own most entries: shared by eight runs'
+// workgroups, the long runs of 1,458 classes at 96 positions made a training
+// step's class sums 606 us instead of 436) and for long runs; past that, with at
+// most 8 partial rows per run on average, 8 runs each: class sums of 20,000
+// entries over 4,000 classes take 20 us instead of 27, of 100,000 over 20,000 57
+// instead of 95, of 200,000 over 100,000 214 instead of 405 (a lane group per run,
+// as before the merge: 24, 63, 217).
 template <typename To>
 int32_t slice_merge(const float* partial, int64_t h, const int64_t* slice_ptr, int64_t n_slices, int64_t n_runs,
                     To* out, hipStream_t s) {
-  if (n_runs >= 1024 && n_slices <= kShort * n_runs) {
+  if (n_runs > 2048 && n_slices <= kShort * n_runs) {
     slice_merge_many_kernel<To><<<unsigned((n_runs + kManyRuns - 1) / kManyRuns), 256, 0, s>>>(
         partial, h, slice_ptr, n_slices, n_runs, out);
     return launched();

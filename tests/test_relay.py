@@ -281,10 +281,10 @@ def test_class_reduce_run_lengths(device, h, dt):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_classes", [1023, 1024, 1031])
+@pytest.mark.parametrize("n_classes", [2048, 2049, 2055])
 @pytest.mark.parametrize("h,odt", [(8, torch.float32), (20, torch.float32), (128, torch.bfloat16), (264, torch.float32)])
 def test_class_reduce_of_many_classes(device, n_classes, h, odt):
-    """Either side of the merge's 1,024 runs and of its 8 runs per workgroup:
+    """Either side of the merge's 2,048 runs and of its 8 runs per workgroup:
     runs of no entry, of one, around 8 partial rows (512 entries) and one that
     owns most entries, the longer ones in one workgroup and apart."""
     gen = torch.Generator().manual_seed(15)
