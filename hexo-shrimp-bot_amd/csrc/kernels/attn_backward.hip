@@ -71,9 +71,10 @@ __device__ __forceinline__ void keep(Chunk8<T>& x, bool ok) {
 // Query-major pass: 16 lanes per query row; up to 16 of its entries are loaded
 // at once, one per lane, and shared by shuffles, so the rows of kB entries are
 // in flight together and their score chains (two head sums and an exponential)
-// run side by side.  Bound by the chain pointers -> indices -> rows and the
-// rows in flight: two entries per step, so that four wavefronts fit a SIMD
-// (64 positions, bf16, 1,075,000 / 416,000 / 416,000 entries: 138 / 112 / 43
+// run side by side.  Bound by the gathered rows' path (TD 75-88% busy, half of it
+// stalled on L1 misses, VALU 52-57%) and the chain pointers -> indices -> rows:
+// two entries per step, so that four wavefronts fit a SIMD, three with fp32 class
+// values (64 positions, bf16, 1,075,000 / 416,000 / 416,000 entries: 138 / 112 / 43
 // us; four entries and a branch per entry 144 / 114 / 42; four side by side,
 // three wavefronts, 143 / 113 / 51; without the q and gradient rows of queries
 // that have no entry 144 / 114 / 43).  With alpha_e, alpha and dalpha of every
@@ -175,6 +176,7 @@ attn_bwd_q_kernel(AttnBwd a, const int64_t* __restrict__ seg_ptr, const int64_t*
   for (int i = 0; i < 8; ++i) d[i] = a.scale * (A[i] - delta * B[i]);
   store8(dq + row * kRow + c0, d);
   if ((lane & 3) == 0) {
+    // (apart too: the class pass reads 16 bytes of it per entry, not 64)
     a.delta[row * kHeads + h] = delta;
     a.stats[row * kHeads + h] = make_float4(mm, inv, delta, 0.f);
     // this lane wrote these entries above: dscore = alpha (dalpha - delta)
@@ -307,7 +309,8 @@ attn_bwd_kv_kernel(AttnBwd a, const int64_t* __restrict__ sseg_ptr, const int64_
 // with qid null dalpha_e already holds it.  16 entries per index load; the gradient
 // rows of kLook entries in flight from clamped indices (a load under a
 // condition is waited for before the next), the scores one entry per lane.
-// Bound by the latency of the gathered gradient rows: with eight rows in
+// Bound by the latency of the gathered gradient rows (TD 67-80% busy, most of it
+// stalled on L1 misses, 10-16% L2 hits, VALU 8%): with eight rows in
 // flight 147 and 53.5 us for 1,075,000 and 416,000 entries (four conditional
 // ones: 156 and 55.6), 22 and 19 for 193,000 and 74,000 (33 and 31).
 template <bool kV>

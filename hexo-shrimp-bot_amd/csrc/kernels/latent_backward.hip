@@ -18,6 +18,10 @@
 // adds the splits' partial sums in split order.  fp32 sums in a fixed order,
 // no atomics: two calls agree bitwise.
 //
+// What bounds the passes is the wavefronts in flight: the broadcast's keeps four
+// latent rows' keys, values and two sums (256 VGPRs, one wavefront per SIMD, TD
+// 45% and VALU 38% busy), the read's half of that (174, two; TD 69%, VALU 49%).
+//
 // (128 positions of 40-120 stones, 169k windows, bf16: forward and backward of
 // the read and the broadcast together 4,810 -> 336 us; before, each operator
 // ran two passes of 1.1 ms over a materialised edge list.)

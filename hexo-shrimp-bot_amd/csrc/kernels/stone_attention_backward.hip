@@ -24,7 +24,7 @@
 // products, exponentials, then 32 or 64 dependent fp32 MFMAs) with two
 // wavefronts per SIMD: MFMA 12-18% busy, VALU 17-18%, half of the wavefronts'
 // time waiting.  192 positions of 44-124 rows, 4 heads of 32, bf16: one row per
-// lane with fp32 FMAs took 74 and 152 us, these passes take 20 and 28; 16
+// lane with fp32 FMAs took 74 and 152 us, these passes take 21 and 26; 16
 // positions of 512-1,024 rows 390 and 611, now 64 and 105.  (Operands cut to
 // bf16 pairs of 16 significant bits: 15 and 17, 40 and 55, but sums that cancel
 // lose those bits and an infinite row turned zeros into NaNs.)
