@@ -112,7 +112,11 @@ __device__ __forceinline__ void store_partial(float (&acc)[kSets][8], float* to)
 template <typename T>
 struct ReadLatents {
   float q[kSlots][8], g[kSlots][8], mm[kSlots], inv[kSlots], delta[kSlots];
-  __device__ __forceinline__ void load(const LatArgs& a, int64_t p, int lane) {
+  // `entries`: the position's run of the order is not empty.  A row of such a
+  // position without a positive l had a score of NaN or +-inf (its output may
+  // be 0 then): delta, the sum of alpha dalpha, is NaN, and so are the row's
+  // dq and its share of dk.
+  __device__ __forceinline__ void load(const LatArgs& a, int64_t p, int lane, bool entries) {
     const int h = lane >> 2;
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
@@ -125,6 +129,7 @@ struct ReadLatents {
       mm[j] = a.m[r * kHeads + h];
       const float ll = a.l[r * kHeads + h];
       inv[j] = ll > 0.f ? 1.f / ll : 0.f;
+      if (entries && !(ll > 0.f)) delta[j] = __builtin_nanf("");
     }
   }
   // one window: its dk, dv, and ds per slot
@@ -152,7 +157,7 @@ latent_read_bwd_kernel(LatArgs a) {
   const int64_t p = blockIdx.x / a.splits;
   const int lane = threadIdx.x % kGroup;
   ReadLatents<T> L;
-  L.load(a, p, lane);
+  L.load(a, p, lane, true);  // (used for the windows of the run only)
   int64_t lo, hi;
   split_range(a, p, int(blockIdx.x % a.splits), lo, hi);
   float acc[kSlots][8];
@@ -211,7 +216,8 @@ struct CastLatents {
       load8(static_cast<const T*>(a.v) + (kSlots * p + j) * a.ldv + 8 * lane, v[j]);
     }
   }
-  // alpha and dalpha of one window, and its delta
+  // alpha and dalpha of one window, and its delta: NaN, as its terms are, for
+  // a window without a positive l (its scores hold a NaN or +-inf)
   __device__ __forceinline__ float terms(const LatArgs& a, const float (&q)[8], const float (&g)[8], float mm,
                                          float ll, float (&al)[kSlots], float (&dd)[kSlots]) const {
     const float inv = ll > 0.f ? 1.f / ll : 0.f;
@@ -223,7 +229,7 @@ struct CastLatents {
       al[j] = inv > 0.f ? expf(sd * a.scale - mm) * inv : 0.f;
       delta = fmaf(al[j], dd[j], delta);
     }
-    return delta;
+    return inv > 0.f ? delta : __builtin_nanf("");
   }
   __device__ __forceinline__ void store_dq(const LatArgs& a, int64_t w, int lane, const float (&ds)[kSlots]) const {
     float d[8];
@@ -378,7 +384,9 @@ latent_bwd_finish_kernel(LatArgs a) {
       float k[8], v[8], dk[8], dv[8], ds[kSlots];
       if (ok) {
         ReadLatents<T> L;
-        L.load(a, p, lane);
+        int64_t st, en;
+        segment(a.offsets, p, a.n_w, st, en);
+        L.load(a, p, lane, en > st);
         load8(static_cast<const T*>(a.k) + w * a.ldk + 8 * lane, k);
         load8(static_cast<const T*>(a.v) + w * a.ldv + 8 * lane, v);
         L.window(a, k, v, dk, dv, ds);

@@ -224,6 +224,42 @@ def test_window_latent_backward_takes_any_order(device):
     mantisnet.ops.raise_on_device_error(device)
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("read", [True, False])
+@pytest.mark.parametrize("which", [0, 1])
+def test_window_latent_backward_keeps_non_finite_scores(device, read, which, value):
+    """A non-finite query or key element: the rows whose softmax it leaves
+    undefined get NaN gradients for all of their head's dims and pass NaN to
+    their head's dims of every key they meet, where autograd through the oracle
+    has NaN; the other positions and heads stay finite.  (Such a row's output
+    can be 0.)"""
+    gen = torch.Generator().manual_seed(33)
+    counts = [70, 0, 3, 18]
+    window_pos = torch.repeat_interleave(torch.arange(4), torch.tensor(counts))
+    window_pos = window_pos[torch.randperm(len(window_pos), generator=gen)]
+    offsets, order = R.window_layout(window_pos, 4)
+    layout = [x.to(device) for x in (window_pos, offsets, order)]
+    sq, sk = ((4, 4, 4, 32), (91, 4, 32)) if read else ((91, 4, 32), (4, 4, 4, 32))
+    ins = [torch.randn(*s, generator=gen) for s in (sq, sk, sk)]
+    # where the forward's own sums are the oracle's: the read's lane groups skip a
+    # NaN score that they meet alone and make a lone -inf a NaN
+    p = 0 if value != value else 2
+    w = int((window_pos == p).nonzero()[1])
+    at = (p, 1, 3, 5) if (which == 0) == read else (w, 3, 5)  # a latent's or a window's head 3
+    ins[which][at] = value
+    go = torch.randn(*sq, generator=gen)
+    op = OPS.window_latent_read if read else OPS.window_latent_broadcast
+    got = _grads(lambda *x: op(*x, *layout)[0], [x.to(device) for x in ins], go.to(device))
+    mantisnet.ops.raise_on_device_error(device)
+    ref = (lambda *x: R.latent_read(*x, offsets, order)) if read else (lambda *x: R.latent_broadcast(*x, window_pos))
+    exp = _grads(ref, ins, go)
+    for g, e in zip(got[:2], exp):
+        assert torch.isnan(e).any() and torch.equal(torch.isnan(g.cpu()), torch.isnan(e))
+    torch.testing.assert_close(got[0].cpu(), exp[0], rtol=1e-4, atol=1e-4, equal_nan=True)
+    torch.testing.assert_close(got[1].cpu(), exp[1], rtol=1e-4, atol=1e-4, equal_nan=True)
+    assert torch.isfinite(got[2]).all()
+
+
 def test_latent_read_backward_without_the_forward_output(device):
     # the module-level call as it was: m, l and the gradient, out formed again
     gen = torch.Generator().manual_seed(28)
